@@ -34,16 +34,17 @@ def workload_params(sgm):
 def path_bytes_per_step(w, h, D, paths, schedule, cost_bytes=1):
     """HBM bytes this build's path sweeps move for one pair (both directions)
     with a uint8 cost volume C, by sweep schedule (the plan's `sweeps`).
-    Path-cost planes (3): the census cost pass writes C (1 B/cell), every
-    direction but the last reads C and writes its plane (1 + 1 B/cell each), the
-    last sweep reads C and the P-1 planes and selects (1 + 7 B/cell): 23 B per
-    cell at 8 paths.  One uint16 aggregate S
+    Excess planes (3): the census cost pass writes C (1 B/cell), the pair sweeps
+    of opposite directions read C twice, write and read a state every 8 steps
+    and write one plane (3.25 B/cell and pair), the winner search reads C and
+    the P/2 planes (1 + 4 B/cell): 19 B per cell at 8 paths.  One uint16
+    aggregate S
     (1, 2): first 1 + 2, middle 1 + 2 + 2 (a paired launch's second member 1 +
     2, and the last sweep then reads both partial sums), last 1 + 2: 36 B per
     cell at 8 paths either way."""
     cells = 2 * w * h * D
     if schedule == 3:
-        per_cell = cost_bytes + (cost_bytes + 1) * (paths - 1) + cost_bytes + (paths - 1)
+        per_cell = cost_bytes + (2 * cost_bytes + 1.25) * (paths // 2) + cost_bytes + paths // 2
     else:
         per_cell = (cost_bytes + 2) + (cost_bytes + 4) * (paths - 2) + (cost_bytes + 2)
     return cells * per_cell
@@ -61,7 +62,7 @@ def algorithmic_bytes_per_step(w, h, D, paths):
 # Sources whose change invalidates the committed HBM traffic measurement of the
 # path sweeps (profiles/path_traffic.json carries the hash it was measured at).
 TRAFFIC_SOURCES = ["pose_amd/csrc/sgm_paths.h", "pose_amd/csrc/sgm_kernels.h",
-                   "pose_amd/csrc/sgm_path_launch.h"]
+                   "pose_amd/csrc/sgm_excess.h", "pose_amd/csrc/sgm_path_launch.h"]
 
 
 def kernel_source_hash():
@@ -660,9 +661,9 @@ def write_traffic(fetch_dir, write_dir, copy_bytes=2 << 30, paths=8):
     then WRITE_SIZE, KiB per dispatch).  Each counter is scaled by what it
     reads for the library's copy kernel (copy_bytes read + copy_bytes written
     per launch); path launches are grouped by kind, and the per-launch figure
-    weights them as one pair does under the schedule the passes ran (path-cost
-    planes: the census cost pass, the P - 1 directions of the planes, the last
-    sweep, one launch each; one aggregate: one first, P - 2 middle, one last)."""
+    weights them as one pair does under the schedule the passes ran (excess
+    planes: the census cost pass, the pair sweeps, the winner search, one launch
+    each; one aggregate: one first, P - 2 middle, one last)."""
     W, H, D = 1600, 1067, 256
     fetch, write = read_counter_csv(fetch_dir, "FETCH_SIZE"), read_counter_csv(write_dir, "WRITE_SIZE")
 
@@ -679,11 +680,12 @@ def write_traffic(fetch_dir, write_dir, copy_bytes=2 << 30, paths=8):
     # the workload's instances only (lane group 4, uint16 aggregates): other
     # legs of the same run launch other lane groups and 32-bit aggregates
     sweep = lambda k, phase: "path_kernel<4, unsigned short, %d, " % phase in k
-    planes = any("path_multi_kernel<4, " in k for k, _ in fetch)
+    planes = any("excess_kernel<16, 16, " in k for k, _ in fetch)
     if planes:
         kinds = (("cost", lambda k: sweep(k, 3), cells, 1),
-                 ("multi", lambda k: "path_multi_kernel<4, " in k, 2 * (paths - 1) * cells, 1),
-                 ("last", lambda k: sweep(k, 2), paths * cells, 1))
+                 ("excess", lambda k: "excess_kernel<16, 16, " in k,
+                  int(3.25 * (paths // 2) * cells), 1),
+                 ("winner", lambda k: "winner_kernel<16, 16, " in k, (1 + paths // 2) * cells, 1))
     else:
         kinds = (("first", lambda k: sweep(k, 0), 3 * cells, 1),
                  ("mid", lambda k: sweep(k, 1), 5 * cells, paths - 2),
@@ -796,7 +798,7 @@ def main():
     kernels = {k: round(v["total_ms"] / args.profile_steps, 4) for k, v in prof.items()}
     # each path launch of the schedule on its own: duration and the build's bytes
     cells = 2 * W * H * D
-    own_bytes = ({"path_cost": 1, "path_multi": 2 * (P - 1), "path_last": 1 + (P - 1)}
+    own_bytes = ({"path_cost": 1, "path_excess": 3.25 * (P // 2), "path_winner": 1 + P // 2}
                  if schedule == 3 else {"path_first": 3, "path_mid": 5, "path_pair": 8, "path_last": 3})
     path_kernels = {}
     for k in path_keys:
@@ -886,7 +888,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": "plain SGM pair 1600x1067, census 9x7, D=256, P1=8 P2=96, "
                                "8 paths, left+right + L-R check; uint8 cost volume, uint8 "
-                               "path-cost planes summed in packed uint16 by the last sweep",
+                               "excess planes summed in packed uint16 by the winner search",
                    "width": W, "height": H, "disparities": D, "paths": P, "pairs_per_step": 1},
         "device": {k: dev[k] for k in ("name", "arch", "memory", "compute_units")},
         "pairs_per_s": round(1e3 / ms_per_step, 3),
@@ -897,15 +899,15 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBPS,
                      "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBPS, 4),
                      "traffic": traffic,
-                     "kernel": "path sweeps of one pair (sgm::path_kernel first and last, "
-                               "sgm::path_multi_kernel for the middle directions)",
+                     "kernel": "path sweeps of one pair (sgm::path_kernel cost pass, "
+                               "sgm::excess_kernel, sgm::winner_kernel)",
                      "sweeps": ["auto", "sequential", "paired", "planes"][schedule],
                      "launches_per_step": path_launches,
                      "launch_ms": round(launch_s * 1e3, 4),
                      "algorithmic_bytes_per_launch": alg_launch,
                      "algorithmic_model": "6P-2 B per cell (uint16 C and S, selection fused "
                                           "into the last sweep), 2*W*H*D cells per pair; the "
-                                          "plane schedule moves 22 B per cell, so the model's "
+                                          "plane schedule moves 19 B per cell, so the model's "
                                           "rate can pass the HBM peak (build_frac is the "
                                           "fraction of peak used)",
                      "path_kernels": path_kernels,

@@ -346,13 +346,15 @@ int sgm_set_cost_volume(sgm_context *ctx, int policy);
  *     its own partial aggregate volume; the last sweep adds both (uint16 sums
  *     wrap modulo 2^16 in any order).  One more aggregate volume per matching
  *     direction.
- *   PLANES: every direction but the last stores its path costs as bytes into a
- *     plane of its own (the middle directions all in one launch, as they only
- *     read the cost volume); the last sweep adds the 7 planes to its own path
- *     costs before the winner search.  A valid cell's path cost is at most its
- *     cost plus P2, so this needs window bits - 1 + P2 <= 255, uint8 costs, 8
- *     paths and no kept volumes; 7 bytes per cell in place of the 2-byte
- *     aggregate, and 22 instead of 36 bytes of HBM traffic per cell.
+ *   PLANES: a path cost is the cell's cost plus an excess of at most P2, so
+ *     every direction, or pair of opposite directions (2 P2 <= 255, large
+ *     pairs), stores its excesses as bytes into a plane of its own, all in one
+ *     launch (they only read the cost volume); the winner search adds the planes
+ *     to the costs.  Needs P2 <= 255, for uint8 costs window bits - 1 + P2 <=
+ *     255, 8 paths, at most 1024 padded disparities and no kept volumes; 8 or 4
+ *     bytes per cell in place of the 2-byte aggregate, and 26 or 19 instead of
+ *     36 bytes of HBM traffic per cell.  (4 paths under PAIRED: the room of the
+ *     two partial aggregates holds one such plane per path.)
  *   AUTO (default): PLANES where it applies and fits the budget, else PAIRED
  *     where that fits, else SEQUENTIAL.  A requested schedule that does not
  *     apply falls back the same way (PLANES -> PAIRED -> SEQUENTIAL). */
@@ -403,7 +405,7 @@ typedef struct sgm_pair {
 /* Phase-major run: one census launch over every image (then the work-queue
  * kernel for the cost items of non-census costs), the path sweeps as launches
  * per lane group of the specialised sweep kernels over a table of all pairs'
- * lines (with path-cost planes: per sub-batch of pairs, lane groups on two
+ * lines (with excess planes: per sub-batch of pairs, lane groups on two
  * streams), then one left-right launch over every pair; all in one graph
  * with SGM_BATCH_GRAPH.  Same results. */
 #define SGM_BATCH_PHASED 8

@@ -792,15 +792,26 @@ CostArgs cost_args(const sgm_params *p) {
   A.gradcap = p->gradient_truncation;
   A.inv_code = invalid_code(p);
   A.u8 = cost_u8(p) ? 1 : 0;
+  A.inv_store = A.pad_store = A.u8 ? 255 : A.inv_code;
   return A;
+}
+
+// Volume codes of the excess-plane kernels (sgm_excess.h).
+void excess_codes(CostArgs &A) {
+  A.inv_store = A.u8 ? 254 : A.inv_code;
+  A.pad_store = A.u8 ? 255 : 0x8FFF;
 }
 
 // Cost rows [J.y0, J.y0 + rows) of every job (rows < 0: the whole image).
 int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h, int Dp,
-                const sgm_params *p, int rows, bool force_u16) {
+                const sgm_params *p, int rows, bool force_u16, bool excess) {
   ProfileScope ps(ctx, "cost");
   CostArgs A = cost_args(p);
-  if (force_u16) A.u8 = 0;
+  if (force_u16) {
+    A.u8 = 0;
+    A.inv_store = A.pad_store = A.inv_code;
+  }
+  if (excess) excess_codes(A);
   const int gy = rows < 0 ? h : rows;
   if (p->cost == SGM_COST_ZNCC || p->cost == SGM_COST_ZNCC_FP32) {
     const int ntx = (w + kZnccTX - 1) / kZnccTX, ntd = (Dp + 63) / 64;
@@ -847,6 +858,27 @@ PathArgs path_args(const sgm_params *p, int dir, int njobs, int total_lines, int
   A.uniq = p->uniqueness;
   A.order = nullptr;
   return A;
+}
+
+// Directions and penalties of an excess launch over `njobs` jobs into `planes`
+// planes per pixel (one per path, or per pair of opposite paths); the caller
+// fills in the waves.
+ExcessArgs excess_args(const sgm_params *p, int njobs, int planes) {
+  ExcessArgs E;
+  memset(&E, 0, sizeof E);
+  E.ndirs = E.planes = planes;
+  E.pairs = planes < p->directions;
+  static const int pair_of[4] = {0, 2, 4, 5};  // with the opposite: 1, 3, 7, 6
+  for (int k = 0; k < E.ndirs; k++) {
+    const PathArgs A = path_args(p, E.pairs ? pair_of[k] : k, njobs, 0, 0);
+    E.dx[k] = A.dx;
+    E.dy[k] = A.dy;
+  }
+  E.p1 = p->p1;
+  E.p2 = effective_p2(p);
+  E.edge = p->edge_scale;
+  E.njobs = njobs;
+  return E;
 }
 
 int lines_of(int cls, int w, int h) { return cls == 0 ? h : cls == 1 ? w : w + h - 1; }
@@ -925,10 +957,12 @@ struct PairBuffers {
   // paired sweeps: the second partial aggregate volume of each matching
   // direction (null: one aggregate, directions swept one per launch)
   void *sum_b[2];
-  // path-cost plane schedule: kPlanes planes of Dp bytes per pixel (interleaved
-  // per pixel) for each matching direction in place of the aggregate (null: an
-  // aggregate volume)
+  // excess planes: nplanes planes of Dp bytes per pixel (interleaved per pixel)
+  // for each matching direction in place of the aggregate (null: an aggregate
+  // volume)
   uint8_t *planes[2];
+  int nplanes;
+  int schedule;  // SGM_SWEEPS_* the buffers are laid out for
   float *disp[2], *checked;
   uint8_t *reasons, *boundary, *reasons_out, *boundary_out, *code;
   unsigned long long *stats;
@@ -959,27 +993,60 @@ struct PairBuffers {
 }  // namespace
 
 // Device bytes a sweep schedule adds to pair_bytes(p, w, h, true): the second
-// partial aggregate volumes of paired sweeps, or the path-cost planes of both
-// matching directions (kPlanes bytes per cell) in place of the aggregates.
+// partial aggregate volumes of paired sweeps, or the excess planes of both
+// matching directions (one byte per cell and plane) in place of the aggregates.
 int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule) {
   const int64_t cells = 2 * (int64_t)w * h * padded_disparities(p->disparities);
   if (schedule == SGM_SWEEPS_PAIRED) return cells * aggregate_bytes(p);
-  if (schedule == SGM_SWEEPS_PLANES) return cells * (kPlanes - aggregate_bytes(p));
+  if (schedule == SGM_SWEEPS_PLANES)
+    return cells * (excess_plane_count(p, cells) - aggregate_bytes(p));
   return 0;
 }
 
-// Whether a multi-direction schedule applies to the pair (budget aside).  Both
-// need packed 16-bit sweeps of lane groups 2..8 over a cost volume.  Path-cost
-// planes also need 8 paths, uint8 costs, no kept volumes (the planes replace
-// the aggregate), and path costs that fit a byte: every valid cell's path cost
-// is at most its cost (<= window bits - 1 for the uint8 costs) plus P2.
-bool sgm::schedule_applies(const sgm_context *ctx, const sgm_params *p, int schedule,
+// Whether the excess-plane kernels (sgm_excess.h) take the pair: excesses that
+// fit a byte (P2 <= 255), a wave shape for the padded range, and lines of a
+// wave whose rows lie within a 32-bit offset of each other.
+bool sgm::excess_possible(const sgm_params *p, int w, int h) {
+  int lanes, R;
+  const int Dp = padded_disparities(p->disparities);
+  return aggregate_bytes(p) == 2 && effective_p2(p) <= 255 && excess_shape(Dp, lanes, R) &&
+         4 * (int64_t)std::max(w, h) * Dp * kMaxExcessDirs < (int64_t)1 << 30;
+}
+
+// Whether a multi-direction schedule applies to the pair (budget aside).
+// Paired sweeps need packed 16-bit sweeps of lane groups 2..8 over a cost
+// volume.  The planes need 8 paths, no kept volumes (the planes replace the
+// aggregate), the excess kernels, and for the uint8 costs a path cost (cost <=
+// window bits - 1, plus P2) that fits a byte.
+bool sgm::schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                            bool cost_volume) {
   if (schedule == SGM_SWEEPS_SEQUENTIAL) return true;
-  if (!cost_volume || aggregate_bytes(p) != 2 || path_lanes(p) > 8) return false;
-  if (schedule == SGM_SWEEPS_PAIRED) return true;
-  return schedule == SGM_SWEEPS_PLANES && !ctx->keep_volumes && cost_u8(p) &&
-         p->directions == kPlanes + 1 && p->window_w * p->window_h - 1 + effective_p2(p) <= 255;
+  if (!cost_volume || aggregate_bytes(p) != 2) return false;
+  if (schedule == SGM_SWEEPS_PAIRED) return path_lanes(p) <= 8;
+  return schedule == SGM_SWEEPS_PLANES && !ctx->keep_volumes && p->directions == kMaxExcessDirs &&
+         excess_possible(p, w, h) &&
+         (!cost_u8(p) || p->window_w * p->window_h - 1 + effective_p2(p) <= 255);
+}
+
+// Planes per pixel of 8 paths over `cells` cells of all matching directions: one
+// per path, or one per pair of opposite paths (PairSweep, sgm_excess.h) where
+// their summed excesses fit a byte and the volumes are so far beyond the caches
+// that HBM traffic counts.
+int sgm::excess_plane_count(const sgm_params *p, int64_t cells) {
+  const bool pairs = 2 * effective_p2(p) <= 255 && cells * (1 + kMaxExcessDirs) > kPairBytes;
+  return pairs ? kMaxExcessDirs / 2 : kMaxExcessDirs;
+}
+
+// Excess planes per pixel of a pair on the resident plan under `schedule` (0:
+// aggregate volumes).  With 4 paths the two partial aggregates of the paired
+// schedule are the room of one plane per path.
+int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule) {
+  if (schedule == SGM_SWEEPS_PLANES)
+    return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities));
+  if (schedule == SGM_SWEEPS_PAIRED && p->directions == 4 && !ctx->keep_volumes &&
+      excess_possible(p, w, h))
+    return 4;
+  return 0;
 }
 
 // Sweep schedule of a resident pair under `budget` (SGM_SWEEPS_SEQUENTIAL,
@@ -992,7 +1059,7 @@ int sgm::sweep_schedule(const sgm_context *ctx, const sgm_params *p, int w, int 
   const int64_t base = pair_bytes(p, w, h, true);
   for (int sched : {SGM_SWEEPS_PLANES, SGM_SWEEPS_PAIRED}) {
     if (sched == SGM_SWEEPS_PLANES && want == SGM_SWEEPS_PAIRED) continue;
-    if (schedule_applies(ctx, p, sched, cost_volume) &&
+    if (schedule_applies(ctx, p, w, h, sched, cost_volume) &&
         base + schedule_bytes(p, w, h, sched) <= budget)
       return sched;
   }
@@ -1003,14 +1070,14 @@ namespace {
 
 // Whole-image device buffers of a pair, by name and size: inputs, descriptors
 // and disparities of both matching directions, the outputs, and (`volumes`)
-// the aggregate volumes (path-cost planes under SGM_SWEEPS_PLANES, a second
-// partial aggregate under SGM_SWEEPS_PAIRED) with (`cost_volume`) the cost
+// the aggregate volumes (`planes` excess planes in their place where not 0, a
+// second partial aggregate under SGM_SWEEPS_PAIRED) with (`cost_volume`) the cost
 // volumes.  Their sum is pair_bytes(p, w, h, cost_volume) (+ schedule_bytes)
 // when `volumes` is set.
 static std::vector<std::pair<std::string, size_t>> pair_buffer_list(const sgm_params *p, int w,
                                                                     int h, bool volumes,
                                                                     bool cost_volume,
-                                                                    int schedule) {
+                                                                    int schedule, int planes) {
   const size_t n = (size_t)w * h, Dp = padded_disparities(p->disparities);
   const int sb = aggregate_bytes(p), words = words_of(p);
   const bool zncc = p->cost == SGM_COST_ZNCC || p->cost == SGM_COST_ZNCC_FP32;
@@ -1027,9 +1094,9 @@ static std::vector<std::pair<std::string, size_t>> pair_buffer_list(const sgm_pa
       L.emplace_back("wsum2" + s, n * 4);
     }
     if (volumes && cost_volume) L.emplace_back("cost" + s, n * Dp * (cost_u8(p) ? 1 : 2));
-    if (volumes && schedule == SGM_SWEEPS_PLANES) L.emplace_back("planes" + s, n * Dp * kPlanes);
+    if (volumes && planes) L.emplace_back("planes" + s, n * Dp * planes);
     else if (volumes) L.emplace_back("sum" + s, n * Dp * sb);
-    if (volumes && schedule == SGM_SWEEPS_PAIRED) L.emplace_back("sumb" + s, n * Dp * sb);
+    if (volumes && !planes && schedule == SGM_SWEEPS_PAIRED) L.emplace_back("sumb" + s, n * Dp * sb);
     L.emplace_back("disp" + s, n * 4);
   }
   L.emplace_back("checked", n * 4);
@@ -1051,7 +1118,8 @@ static std::vector<std::pair<std::string, size_t>> pair_buffer_list(const sgm_pa
 int64_t sgm::resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h,
                                 bool cost_volume, int schedule, bool fresh) {
   int64_t total = fresh ? 0 : ctx->allocated;
-  for (const auto &b : pair_buffer_list(p, w, h, true, cost_volume, schedule)) {
+  const int planes = excess_planes(ctx, p, w, h, schedule);
+  for (const auto &b : pair_buffer_list(p, w, h, true, cost_volume, schedule, planes)) {
     if (fresh) {
       total += (int64_t)b.second;
       continue;
@@ -1075,6 +1143,7 @@ int ensure_pair_buffers(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
   const bool recompute = !rows && recompute_cost(ctx, p, w, h);
   const int schedule =
       rows ? SGM_SWEEPS_SEQUENTIAL : sweep_schedule(ctx, p, w, h, !recompute, ctx->budget);
+  const int planes = excess_planes(ctx, p, w, h, schedule);
   int rc;
 #define ENSURE(name, bytes)                                                   \
   if ((rc = ctx->buffers[name].ensure(ctx, (bytes), name)) != SGM_OK) return rc;
@@ -1083,13 +1152,13 @@ int ensure_pair_buffers(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
     // the streamed and compact plans hold no whole-image volume
     for (const char *v : {"cost0", "cost1", "sum0", "sum1"}) ctx->buffers[v].release(ctx);
   }
-  if (schedule != SGM_SWEEPS_PAIRED)
+  if (schedule != SGM_SWEEPS_PAIRED || planes)
     for (const char *v : {"sumb0", "sumb1"}) ctx->buffers[v].release(ctx);
-  if (schedule != SGM_SWEEPS_PLANES)
+  if (!planes)
     for (const char *v : {"planes0", "planes1"}) ctx->buffers[v].release(ctx);
   else
     for (const char *v : {"sum0", "sum1"}) ctx->buffers[v].release(ctx);
-  for (const auto &b : pair_buffer_list(p, w, h, rows == 0, !recompute, schedule))
+  for (const auto &b : pair_buffer_list(p, w, h, rows == 0, !recompute, schedule, planes))
     ENSURE(b.first.c_str(), b.second);
   for (int d = 0; d < 2; d++) {
     const std::string s = std::to_string(d);
@@ -1102,12 +1171,14 @@ int ensure_pair_buffers(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
     B.wsum2[d] = zncc ? (int32_t *)ctx->buffers["wsum2" + s].ptr : nullptr;
     B.cost[d] = rows || recompute ? nullptr : (uint16_t *)ctx->buffers["cost" + s].ptr;
     B.recompute = recompute;
-    B.sum[d] = rows || schedule == SGM_SWEEPS_PLANES ? nullptr : ctx->buffers["sum" + s].ptr;
-    B.sum_b[d] = schedule == SGM_SWEEPS_PAIRED ? ctx->buffers["sumb" + s].ptr : nullptr;
-    B.planes[d] =
-        schedule == SGM_SWEEPS_PLANES ? (uint8_t *)ctx->buffers["planes" + s].ptr : nullptr;
+    B.sum[d] = rows || planes ? nullptr : ctx->buffers["sum" + s].ptr;
+    B.sum_b[d] =
+        schedule == SGM_SWEEPS_PAIRED && !planes ? ctx->buffers["sumb" + s].ptr : nullptr;
+    B.planes[d] = planes ? (uint8_t *)ctx->buffers["planes" + s].ptr : nullptr;
     B.disp[d] = (float *)ctx->buffers["disp" + s].ptr;
   }
+  B.nplanes = planes;
+  B.schedule = schedule;
   B.bgr[0] = B.bgr[1] = nullptr;
   B.refine = nullptr;
   B.strip_rows = pool ? 0 : rows;
@@ -1567,6 +1638,14 @@ int line_length(int dx, int dy, int line, int w, int h) {
   return std::min(dx > 0 ? w - x : x + 1, dy > 0 ? h - y : y + 1);
 }
 
+int wave_length(int dx, int dy, int wave, int per, int w, int h) {
+  const int lines = lines_of(dy == 0 ? 0 : dx == 0 ? 1 : 2, w, h);
+  int n = 0;
+  for (int l = wave * per; l < std::min(lines, (wave + 1) * per); l++)
+    n = std::max(n, line_length(dx, dy, l, w, h));
+  return n;
+}
+
 void longest_first(const std::vector<int> &len, int maxlen, std::vector<int> &order) {
   // counting sort by length, descending; lines of equal length in line order
   std::vector<int> start((size_t)maxlen + 2, 0);
@@ -1580,18 +1659,19 @@ void longest_first(const std::vector<int> &len, int maxlen, std::vector<int> &or
 
 namespace {
 
-// Longest-first dispatch order of the lines of a launch over a w x h pair (nd
-// matching directions; lines [begin[k], begin[k] + nd * split[k]) sweep
-// direction (dx[k], dy[k]), matching direction m's from begin[k] + m *
-// split[k]), in a device buffer cached by shape.  A launch with several times
-// more lines than resident waves otherwise ends on long lines dispatched last
-// (the seven-direction launch at 1600x1067 D=256: 2.48 -> 2.30 ms).  Null, for
-// the natural order, when the buffer does not fit the budget.
+// Longest-first dispatch order of the waves of a launch over a w x h pair (nd
+// matching directions; waves [begin[k], begin[k] + nd * split[k]) sweep
+// direction (dx[k], dy[k]), `per` neighbouring lines each, matching direction
+// m's from begin[k] + m * split[k]), in a device buffer cached by shape.  A
+// launch with several times more lines than resident waves otherwise ends on
+// long lines dispatched last (seven directions with one line per wave at
+// 1600x1067 D=256: 2.48 -> 2.30 ms).  Null, for the natural order, when the
+// buffer does not fit the budget.
 static const int *line_order(sgm_context *ctx, const char *name, int ndirs, const int *dx,
                              const int *dy, const int *split, const int *begin, int total, int w,
-                             int h, int nd) {
+                             int h, int nd, int per = 1) {
   sgm_context::LineOrder &lo = ctx->line_orders[name];
-  const int key[6] = {w, h, nd, ndirs, dx[0], dy[0]};
+  const int key[7] = {w, h, nd, ndirs, dx[0], dy[0], per};
   Buffer &buf = ctx->buffers[name];
   if (buf.ptr && memcmp(lo.key, key, sizeof key) == 0) return (const int *)buf.ptr;
   const size_t bytes = (size_t)total * sizeof(int);
@@ -1602,7 +1682,7 @@ static const int *line_order(sgm_context *ctx, const char *name, int ndirs, cons
   for (int k = 0; k < ndirs; k++)
     for (int m = 0; m < nd; m++)
       for (int l = 0; l < split[k]; l++)
-        len[(size_t)begin[k] + (size_t)m * split[k] + l] = line_length(dx[k], dy[k], l, w, h);
+        len[(size_t)begin[k] + (size_t)m * split[k] + l] = wave_length(dx[k], dy[k], l, per, w, h);
   longest_first(len, std::max(w, h), lo.host);
   hipError_t e = hipMemcpyAsync(buf.ptr, lo.host.data(), bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e != hipSuccess) {
@@ -1882,7 +1962,7 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
       J.minD = p->min_disparity;
       J.reverse = d;
     }
-    if ((rc = launch_cost(ctx, cj, nd, w, h, Dp, p))) return rc;
+    if ((rc = launch_cost(ctx, cj, nd, w, h, Dp, p, -1, false, B.nplanes > 0))) return rc;
   }
   PathJobs pj;
   memset(&pj, 0, sizeof pj);
@@ -1925,45 +2005,39 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     (void)hipStreamSynchronize(ctx->stream);
     return true;
   };
-  if (B.planes[slots[0]] && (mode & 7) == 4) {
-    // Path-cost planes: the census cost pass (fused census cost of the
-    // left-to-right lines; other costs come from the cost kernel above), every
-    // direction but the last in one launch, each into its plane 0..6, and the
-    // last sweep, which adds the seven planes to its own path costs before the
-    // winner search.
-    ctx->last_sweeps = SGM_SWEEPS_PLANES;
+  if (B.nplanes) {
+    // Excess planes: the census cost pass (fused census cost; other costs come
+    // from the cost kernel above), every direction in one launch, each into its
+    // plane, and the winner search over the planes.
+    ctx->last_sweeps = B.schedule;
+    const int cost_bytes = cost_u8(p) ? 1 : 2;
+    const bool stream = (int64_t)nd * w * h * Dp * (cost_bytes + B.nplanes) > kStreamBytes;
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
     if (fused) {
       PathArgs Ac = dir_args(0);
       Ac.split = h * cost_segments(w);
       Ac.total_lines = nd * Ac.split;
-      if ((rc = launch_path(ctx, R, sb, 2 | (mode & MODE_NT), pj, Ac, PHASE_COST, waves))) return rc;
+      if ((rc = launch_path(ctx, R, sb, 2 | (stream ? MODE_NT : 0), pj, Ac, PHASE_COST, waves)))
+        return rc;
     }
-    MultiDir M;
-    memset(&M, 0, sizeof M);
-    M.ndirs = p->directions - 1;
-    for (int k = 0; k < M.ndirs; k++) {
-      const PathArgs Ak = dir_args(k);
-      M.dx[k] = Ak.dx;
-      M.dy[k] = Ak.dy;
-      M.cls[k] = Ak.cls;
-      M.split[k] = Ak.split;
-      M.begin[k] = M.total_lines;
-      M.total_lines += Ak.total_lines;
-      for (int i = 0; i < nd; i++) M.plane[k][i] = B.planes[slots[i]] + (size_t)k * Dp;
+    for (int i = 0; i < nd; i++) pj.local[i].sum = B.planes[slots[i]];
+    ExcessArgs E = excess_args(p, nd, B.nplanes);
+    int lanes = 0, er = 0;
+    excess_shape(Dp, lanes, er);
+    const int per = 64 / lanes;
+    for (int k = 0; k < E.ndirs; k++) {
+      const int cls = E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2;
+      E.split[k] = (lines_of(cls, w, h) + per - 1) / per;
+      E.begin[k] = E.total;
+      E.total += nd * E.split[k];
     }
-    M.order = line_order(ctx, "multi_order", M.ndirs, M.dx, M.dy, M.split, M.begin, M.total_lines,
-                         w, h, nd);
+    E.order = line_order(ctx, "excess_order", E.ndirs, E.dx, E.dy, E.split, E.begin, E.total, w, h,
+                         nd, per);
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
-    if ((rc = launch_path_multi(ctx, R, mode | MODE_PLANE, pj, dir_args(0), M, waves))) return rc;
-    PathJobs jl = pj;
-    for (int i = 0; i < nd; i++) jl.local[i].sum = B.planes[slots[i]];
+    if ((rc = launch_excess(ctx, Dp, cost_bytes, stream, pj, E))) return rc;
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
-    PathArgs AL = dir_args(p->directions - 1);
-    const int zero = 0;
-    AL.order = line_order(ctx, "last_order", 1, &AL.dx, &AL.dy, &AL.split, &zero, AL.total_lines, w,
-                          h, nd);
-    return launch_path(ctx, R, sb, mode | MODE_PLANE, jl, AL, PHASE_LAST, waves);
+    return launch_winner(ctx, Dp, cost_bytes, B.nplanes, E.pairs ? 2 * E.p2 : E.p2, stream, pj,
+                         WinnerArgs{p->directions, p->uniqueness}, w, h, nd);
   }
   // Paired sweeps: after the first direction, the middle directions run two
   // per launch, the first of each pair adding into the aggregate volume and

@@ -85,81 +85,86 @@ static size_t group_table_bound(int count) {
 // in one device allocation.
 static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sgm_pair *pairs,
                         int count) {
-  std::vector<int> rs;
+  // a group: one lane group R, under excess planes one wave shape of them
+  auto shape_of = [&](const PathJob &J) {
+    int lanes = 0, er = 0;
+    if (b->planes) excess_shape(J.Dp, lanes, er);
+    return std::make_pair(J.R, lanes * 64 + er);
+  };
+  std::vector<std::pair<int, int>> rs;
   for (const PathJob &J : jobs)
-    if (std::find(rs.begin(), rs.end(), J.R) == rs.end()) rs.push_back(J.R);
+    if (std::find(rs.begin(), rs.end(), shape_of(J)) == rs.end()) rs.push_back(shape_of(J));
   std::sort(rs.begin(), rs.end());
   const int sb = b->sum_bytes;
   std::vector<uint8_t> host;
   struct Pending {
-    size_t jobs_off, lb_off[4], multi_off = 0, last_off = 0;
+    size_t jobs_off, lb_off[4], order_off = 0;
   };
   std::vector<Pending> offs;
   b->groups.clear();
-  // sub-batch by sub-batch (path-cost planes reuse one scratch region), and
-  // within a sub-batch one group per lane group R
+  // sub-batch by sub-batch (excess planes reuse one scratch region), and
+  // within a sub-batch group by group
   for (int sub = 0; sub < b->nsub; sub++)
-  for (int R : rs) {
+  for (const std::pair<int, int> &key : rs) {
+    const int R = key.first;
     sgm_batch::Group g;
     g.R = R;
     g.sub = sub;
+    const int per = b->planes ? 64 / (key.second / 64) : 1;  // lines per wave
     std::vector<PathJob> gj;
     int64_t volume = 0;
     bool aligned = true;
     for (size_t j = 0; j < jobs.size(); j++) {
       const PathJob &J = jobs[j];
-      if (J.R == R && b->pair_sub[j / 2] == sub) {
+      if (shape_of(J) == key && b->pair_sub[j / 2] == sub) {
         gj.push_back(J);
-        volume += (int64_t)J.w * J.h * J.Dp * (b->cost8 ? 3 : 4);
+        volume += (int64_t)J.w * J.h * J.Dp *
+                  (b->planes ? 1 + b->nplanes : b->cost8 ? 3 : 4);
         aligned &= J.Dp % 64 == 0;
+        g.Dp = J.Dp;
+        g.w = std::max(g.w, J.w);
+        g.h = std::max(g.h, J.h);
       }
     }
     if (gj.empty()) continue;
     g.njobs = (int)gj.size();
     // stream the volumes past the caches as the plain path does: whole 64-byte
     // lines only, volumes far beyond the 256 MB MALL
-    g.nt = sb == 2 && !b->recompute && aligned && R <= 8 && volume > ((int64_t)768 << 20);
+    g.nt = b->planes ? volume > kStreamBytes
+                     : sb == 2 && !b->recompute && aligned && R <= 8 && volume > ((int64_t)768 << 20);
     Pending pd;
     pd.jobs_off = align_up(host.size(), 256);
     host.resize(pd.jobs_off + gj.size() * sizeof(PathJob));
     memcpy(host.data() + pd.jobs_off, gj.data(), gj.size() * sizeof(PathJob));
     for (int cls = 0; cls < 4; cls++) {
-      // line classes 0..2, and 3: the row segments of the census cost pass
+      // the waves of line classes 0..2, and 3: the row segments of the census
+      // cost pass
       std::vector<int> lb(gj.size() + 1, 0);
       for (size_t j = 0; j < gj.size(); j++)
         lb[j + 1] = lb[j] + (cls == 3 ? gj[j].h * cost_segments(gj[j].w)
-                                      : lines_of(cls, gj[j].w, gj[j].h));
+                                      : (lines_of(cls, gj[j].w, gj[j].h) + per - 1) / per);
       g.total_lines[cls] = lb.back();
       pd.lb_off[cls] = align_up(host.size(), 256);
       host.resize(pd.lb_off[cls] + lb.size() * sizeof(int));
       memcpy(host.data() + pd.lb_off[cls], lb.data(), lb.size() * sizeof(int));
     }
     if (b->planes && !b->external) {
-      // longest-first orders (as the plain path's): the directions but the
-      // last in one launch, each over every job's lines of its class, then
-      // the last direction alone
-      static const int dirs[8][2] = {{1, 0}, {-1, 0}, {0, 1}, {0, -1}, {1, 1}, {-1, 1}, {1, -1}, {-1, -1}};
-      const int P = b->params.directions;
+      // longest-first order, as the plain path's: every direction in one
+      // launch, each over every job's waves of its class
+      const ExcessArgs E = excess_args(&b->params, g.njobs, b->nplanes);
       int maxlen = 1;
       for (const PathJob &J : gj) maxlen = std::max(maxlen, std::max(J.w, J.h));
-      auto lengths = [&](int dir, std::vector<int> &len) {
-        const int dx = dirs[dir][0], dy = dirs[dir][1];
-        const int cls = dy == 0 ? 0 : dx == 0 ? 1 : 2;
-        for (const PathJob &J : gj)
-          for (int l = 0; l < lines_of(cls, J.w, J.h); l++) len.push_back(line_length(dx, dy, l, J.w, J.h));
-      };
       std::vector<int> len, order;
-      for (int d = 0; d < P - 1; d++) lengths(d, len);  // the launch's line numbering
+      for (int k = 0; k < E.ndirs; k++)
+        for (const PathJob &J : gj) {
+          const int lines = lines_of(E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2, J.w, J.h);
+          for (int l = 0; l * per < lines; l++)
+            len.push_back(wave_length(E.dx[k], E.dy[k], l, per, J.w, J.h));
+        }
       longest_first(len, maxlen, order);
-      pd.multi_off = align_up(host.size(), 256);
-      host.resize(pd.multi_off + order.size() * sizeof(int));
-      memcpy(host.data() + pd.multi_off, order.data(), order.size() * sizeof(int));
-      len.clear();
-      lengths(P - 1, len);
-      longest_first(len, maxlen, order);
-      pd.last_off = align_up(host.size(), 256);
-      host.resize(pd.last_off + order.size() * sizeof(int));
-      memcpy(host.data() + pd.last_off, order.data(), order.size() * sizeof(int));
+      pd.order_off = align_up(host.size(), 256);
+      host.resize(pd.order_off + order.size() * sizeof(int));
+      memcpy(host.data() + pd.order_off, order.data(), order.size() * sizeof(int));
     }
     offs.push_back(pd);
     b->groups.push_back(g);
@@ -183,10 +188,7 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
   for (size_t i = 0; i < b->groups.size(); i++) {
     b->groups[i].jobs = (const PathJob *)(base + offs[i].jobs_off);
     for (int cls = 0; cls < 4; cls++) b->groups[i].line_begin[cls] = (const int *)(base + offs[i].lb_off[cls]);
-    if (offs[i].multi_off) {
-      b->groups[i].order_multi = (const int *)(base + offs[i].multi_off);
-      b->groups[i].order_last = (const int *)(base + offs[i].last_off);
-    }
+    if (offs[i].order_off) b->groups[i].order = (const int *)(base + offs[i].order_off);
   }
   b->phased = true;
   return SGM_OK;
@@ -247,10 +249,9 @@ static int phased_enqueue(sgm_batch *b) {
   if ((rc = queue_launch(b, pb[BPH_COST], pb[BPH_PATH0], b->args.head, "batch cost"))) return rc;
   const int sb = b->sum_bytes;
   if (b->planes) {
-    // path-cost planes, sub-batch after sub-batch (one scratch region): per
-    // lane group the census cost pass, every direction but the last in one
-    // launch (planes 0..6), the last sweep over the planes.  With a side
-    // stream, the lane groups of a sub-batch alternate between the two
+    // excess planes, sub-batch after sub-batch (one scratch region): per group
+    // the census cost pass, every direction in one launch, the winner search.
+    // With a side stream, the groups of a sub-batch alternate between the two
     // streams, so one group's launches fill the tail of the other's.
     int cur_sub = -1, gi = 0;
     auto sync_streams = [&](bool fork) -> int {
@@ -273,43 +274,25 @@ static int phased_enqueue(sgm_batch *b) {
         gi = 0;
       }
       hipStream_t st = (b->side && (gi++ & 1)) ? b->side : b->stream;
-      const int nt = g.nt ? MODE_NT : 0;
-      auto args = [&](int dir) {
-        PathArgs A = path_args(p, dir, g.njobs, 0, 0);
-        A.total_lines = g.total_lines[A.cls];
-        return A;
-      };
       PathJobs pj;
       memset(&pj, 0, sizeof pj);
       pj.table = g.jobs;
-      PathArgs Ac = args(0);
+      PathArgs Ac = path_args(p, 0, g.njobs, 0, 0);
       Ac.total_lines = g.total_lines[3];
       pj.line_begin = g.line_begin[3];  // row segments of the cost pass
-      if ((rc = launch_path(ctx, g.R, sb, 2 | nt, pj, Ac, PHASE_COST, path_waves(ctx, g.R), st)))
-        return rc;
-      MultiDir M;
-      memset(&M, 0, sizeof M);
-      M.ndirs = p->directions - 1;
-      for (int k = 0; k < M.ndirs; k++) {
-        const PathArgs Ak = args(k);
-        M.dx[k] = Ak.dx;
-        M.dy[k] = Ak.dy;
-        M.cls[k] = Ak.cls;
-        M.begin[k] = M.total_lines;
-        M.total_lines += Ak.total_lines;
-      }
-      for (int cls = 0; cls < 3; cls++) M.line_begin[cls] = g.line_begin[cls];
-      M.njobs = g.njobs;
-      M.plane0 = 0;
-      M.order = g.order_multi;
-      if ((rc = launch_path_multi(ctx, g.R, 4 | nt | MODE_PLANE, pj, args(0), M,
-                                  path_waves(ctx, g.R), st)))
-        return rc;
-      PathArgs AL = args(p->directions - 1);
-      AL.order = g.order_last;
-      pj.line_begin = g.line_begin[AL.cls];
-      if ((rc = launch_path(ctx, g.R, sb, 4 | nt | MODE_PLANE, pj, AL, PHASE_LAST,
+      if ((rc = launch_path(ctx, g.R, sb, 2 | (g.nt ? MODE_NT : 0), pj, Ac, PHASE_COST,
                             path_waves(ctx, g.R), st)))
+        return rc;
+      ExcessArgs E = excess_args(p, g.njobs, b->nplanes);
+      for (int k = 0; k < E.ndirs; k++) {
+        E.begin[k] = E.total;
+        E.total += g.total_lines[E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2];
+      }
+      for (int cls = 0; cls < 3; cls++) E.wave_begin[cls] = g.line_begin[cls];
+      E.order = g.order;
+      if ((rc = launch_excess(ctx, g.Dp, 1, g.nt, pj, E, st))) return rc;
+      if ((rc = launch_winner(ctx, g.Dp, 1, E.planes, E.pairs ? 2 * E.p2 : E.p2, g.nt, pj,
+                              WinnerArgs{p->directions, p->uniqueness}, g.w, g.h, g.njobs, st)))
         return rc;
     }
     if ((rc = sync_streams(false))) return rc;
@@ -421,22 +404,35 @@ bool batch_recompute_possible(const sgm_params *params, bool keep_volumes) {
          aggregate_bytes(params) == 2;
 }
 
-// Path-cost planes in a phase-major batch: the plain plan's plane conditions
-// with the census cost fused into the first sweep (1-word Census, 16-bit sums).
-bool batch_planes_possible(const sgm_context *ctx, const sgm_params *params, int flags) {
-  return (flags & SGM_BATCH_PHASED) && params->cost == SGM_COST_CENSUS && words_of(params) == 1 &&
-         aggregate_bytes(params) == 2 && params->directions == kPlanes + 1 &&
-         !ctx->keep_volumes &&
-         params->window_w * params->window_h - 1 + effective_p2(params) <= 255 &&
-         (ctx->sweeps == SGM_SWEEPS_AUTO || ctx->sweeps == SGM_SWEEPS_PLANES);
+// Excess planes in a phase-major batch: the plain plan's plane conditions with
+// the fused census cost (1-word Census, 16-bit sums), for every pair.
+bool batch_planes_possible(const sgm_context *ctx, const sgm_params *params, const sgm_pair *pairs,
+                           int count, int flags) {
+  if (!(flags & SGM_BATCH_PHASED) || params->cost != SGM_COST_CENSUS || words_of(params) != 1 ||
+      (ctx->sweeps != SGM_SWEEPS_AUTO && ctx->sweeps != SGM_SWEEPS_PLANES))
+    return false;
+  for (int i = 0; i < count; i++) {
+    sgm_params q = *params;
+    q.disparities = pairs[i].disparities;
+    if (!schedule_applies(ctx, &q, pairs[i].width, pairs[i].height, SGM_SWEEPS_PLANES, true))
+      return false;
+  }
+  return true;
 }
 
-// Scratch bytes of one pair under path-cost planes (carved as batch_create
-// carves them): the uint8 cost volume and the plane block of both matching
-// directions.
-size_t batch_plane_bytes(const sgm_pair &pr) {
+// Excess planes per pixel of a batch.
+int batch_plane_count(const sgm_params *params, const sgm_pair *pairs, int count) {
+  int64_t cells = 0;
+  for (int i = 0; i < count; i++)
+    cells += 2 * (int64_t)pairs[i].width * pairs[i].height * padded_disparities(pairs[i].disparities);
+  return excess_plane_count(params, cells);
+}
+
+// Scratch bytes of one pair under `nplanes` excess planes (carved as batch_create
+// carves them): the uint8 cost volume and the planes of both matching directions.
+size_t batch_plane_bytes(const sgm_pair &pr, int nplanes) {
   const size_t n = (size_t)pr.width * pr.height, Dp = padded_disparities(pr.disparities);
-  return 2 * (align_up(n * Dp, 256) + align_up(n * Dp * kPlanes, 256));
+  return 2 * (align_up(n * Dp, 256) + align_up(n * Dp * nplanes, 256));
 }
 
 size_t batch_arena_bytes(const sgm_params *params, const sgm_pair *pairs, int count, int flags,
@@ -477,8 +473,10 @@ size_t batch_arena_bytes(const sgm_params *params, const sgm_pair *pairs, int co
     if (host_io && pr.reasons) cv.take(n);
     if (host_io && pr.boundary) cv.take(n);
   }
-  if (planes)
-    for (int i = 0; i < count; i++) cv.off += batch_plane_bytes(pairs[i]);
+  if (planes) {
+    const int nplanes = batch_plane_count(params, pairs, count);
+    for (int i = 0; i < count; i++) cv.off += batch_plane_bytes(pairs[i], nplanes);
+  }
   return cv.off;
 }
 
@@ -538,18 +536,19 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
   b->cost8 = !b->recompute && batch_cost8(params);
   b->fused = !b->recompute && params->cost == SGM_COST_CENSUS && b->words == 1 &&
              b->sum_bytes == 2;
-  // Path-cost planes (phase-major runs of the fused census cost): no resident
+  // Excess planes (phase-major runs of the fused census cost): no resident
   // cost or aggregate volume per pair; the cost volumes and plane blocks of a
   // sub-batch of pairs live in one scratch region that the sub-batches reuse
   // in turn.  planes = 1: all pairs in one sub-batch; -1: sub-batches as large
   // as the memory at hand allows (off when not even the largest pair fits).
   b->nsub = 1;
   b->pair_sub.assign(count, 0);
-  if (planes != 0 && b->fused && batch_planes_possible(ctx, params, flags)) {
+  if (planes != 0 && b->fused && batch_planes_possible(ctx, params, pairs, count, flags)) {
+    b->nplanes = batch_plane_count(params, pairs, count);
     size_t total = 0, largest = 0;
     for (int i = 0; i < count; i++) {
-      total += batch_plane_bytes(pairs[i]);
-      largest = std::max(largest, batch_plane_bytes(pairs[i]));
+      total += batch_plane_bytes(pairs[i], b->nplanes);
+      largest = std::max(largest, batch_plane_bytes(pairs[i], b->nplanes));
     }
     size_t cap = total;
     if (planes < 0) {
@@ -564,7 +563,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
       size_t used = 0;
       int sub = 0;
       for (int i = 0; i < count; i++) {
-        const size_t need = batch_plane_bytes(pairs[i]);
+        const size_t need = batch_plane_bytes(pairs[i], b->nplanes);
         if (used + need > cap) {
           sub++;
           used = 0;
@@ -644,7 +643,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
       sc.off = at;
       for (int d = 0; d < 2; d++) {
         offs[i].cost[d] = sc.take(n * Dp);
-        offs[i].sum[d] = sc.take(n * Dp * kPlanes);
+        offs[i].sum[d] = sc.take(n * Dp * b->nplanes);
       }
       at = sc.off;
     }

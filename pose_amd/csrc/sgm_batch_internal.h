@@ -20,12 +20,12 @@ struct PairSlots {
 bool batch_recompute_possible(const sgm_params *params, bool keep_volumes);
 size_t batch_arena_bytes(const sgm_params *params, const sgm_pair *pairs, int count, int flags,
                          bool recompute, bool planes);
-bool batch_planes_possible(const sgm_context *ctx, const sgm_params *params, int flags);
-size_t batch_plane_bytes(const sgm_pair &pr);
+bool batch_planes_possible(const sgm_context *ctx, const sgm_params *params, const sgm_pair *pairs,
+                           int count, int flags);
 size_t batch_table_bytes(int count, const sgm_params *params);
 // recompute: 1 census cost recomputed in the sweeps (no cost volume), 0 resident
 // cost volume, -1 chosen by the context's policy and the memory at hand.
-// planes (phase-major runs): 1 path-cost planes with every pair in one
+// planes (phase-major runs): 1 excess planes with every pair in one
 // sub-batch, 0 one aggregate volume per pair, -1 planes in sub-batches as
 // large as the memory at hand allows, where they apply.
 int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pairs, int count,
@@ -77,17 +77,19 @@ struct sgm_batch {
     int R = 0, njobs = 0, sub = 0;
     bool nt = false;
     const sgm::PathJob *jobs = nullptr;
-    // per line class (horizontal, vertical, diagonal, cost-pass row segments)
+    int Dp = 0, w = 0, h = 0;  // padded disparities of a job, largest sizes
+    // waves per line class (horizontal, vertical, diagonal, cost-pass row segments)
     const int *line_begin[4] = {nullptr, nullptr, nullptr, nullptr};
     int total_lines[4] = {0, 0, 0, 0};
-    // plane runs of non-serving batches: longest-first line orders of the
-    // seven-direction launch and of the last sweep (null: line order)
-    const int *order_multi = nullptr, *order_last = nullptr;
+    // plane runs of non-serving batches: longest-first order of the waves of the
+    // sweeps' launch (null: line order)
+    const int *order = nullptr;
   };
   bool phased = false;
-  // path-cost planes: the scratch region of a sub-batch's cost volumes and
+  // excess planes: the scratch region of a sub-batch's cost volumes and
   // plane blocks, each pair's sub-batch, and the sub-batch count
   bool planes = false;
+  int nplanes = 0;  // excess planes per pixel
   size_t scratch_bytes = 0;
   std::vector<int> pair_sub;
   int nsub = 1;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -65,13 +66,19 @@ int64_t pair_bytes(const sgm_params *p, int w, int h);
 int64_t pair_bytes(const sgm_params *p, int w, int h, bool cost_volume);
 int64_t resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                            int schedule, bool fresh);
-bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int schedule, bool cost_volume);
+bool excess_possible(const sgm_params *p, int w, int h);
+int excess_plane_count(const sgm_params *p, int64_t cells);
+int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule);
+bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
+                      bool cost_volume);
 int64_t schedule_bytes(const sgm_params *p, int w, int h, int schedule);
 int sweep_schedule(const sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                    int64_t budget);
 int lines_of(int cls, int w, int h);
 // length of line `line` of direction (dx, dy) in a w x h image (line_start)
 int line_length(int dx, int dy, int line, int w, int h);
+// longest of the `per` lines of wave `wave`
+int wave_length(int dx, int dy, int wave, int per, int w, int h);
 // the indices of `len` by length, longest first, equal lengths in index order
 void longest_first(const std::vector<int> &len, int maxlen, std::vector<int> &order);
 struct HostCopy {
@@ -101,7 +108,7 @@ int launch_fill_u64(sgm_context *ctx, unsigned long long *p, unsigned long long 
 int launch_census(sgm_context *ctx, const CensusJobs &jobs, int njobs, int w, int h,
                   const sgm_params *p);
 int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h, int Dp,
-                const sgm_params *p, int rows = -1, bool force_u16 = false);
+                const sgm_params *p, int rows = -1, bool force_u16 = false, bool excess = false);
 int64_t streamed_pair_bytes(const sgm_params *p, int w, int h, int rows);
 int64_t streamed_host_bytes(const sgm_params *p, int w, int h);
 int streamed_rows(sgm_context *ctx, const sgm_params *p, int w, int h);
@@ -111,6 +118,11 @@ int64_t esgm_pair_bytes(const sgm_params *p, int w, int h, int rows, int pool);
 const char *esgm_unsupported(const sgm_params *p, int w, int h);
 int esgm_plan(sgm_context *ctx, const sgm_params *p, int w, int h, int *rows, int *pool);
 CostArgs cost_args(const sgm_params *p);
+void excess_codes(CostArgs &A);
+ExcessArgs excess_args(const sgm_params *p, int njobs, int planes);
+// volumes beyond this stream past the caches (far more than the 256 MB MALL)
+constexpr int64_t kStreamBytes = (int64_t)1 << 30;
+constexpr int64_t kPairBytes = (int64_t)1 << 30;
 PathArgs path_args(const sgm_params *p, int dir, int njobs, int total_lines, int keep_sum);
 // on `stream` (the context's stream when null)
 int launch_path(sgm_context *ctx, int R, int sum_bytes, int mode, const PathJobs &jobs,
@@ -121,9 +133,14 @@ int launch_check(const char *what);
 int launch_path_pair(sgm_context *ctx, int R, int mode, int phase_b, const PathJobs &ja,
                      const PathArgs &A, const PathJobs &jb, const PathArgs &B, int waves,
                      hipStream_t stream = nullptr);
-// the directions of `M` in one launch, each storing its path-cost plane
-int launch_path_multi(sgm_context *ctx, int R, int mode, const PathJobs &jobs, const PathArgs &A,
-                      const MultiDir &M, int waves, hipStream_t stream = nullptr);
+// every direction of `A`, each storing its excess plane (sgm_excess.h)
+int launch_excess(sgm_context *ctx, int Dp, int cost_bytes, bool nt, const PathJobs &jobs,
+                  const ExcessArgs &A, hipStream_t stream = nullptr);
+// winner search over `planes` plane rows per pixel, each at most `largest`;
+// w, h: the largest image of the `njobs` jobs
+int launch_winner(sgm_context *ctx, int Dp, int cost_bytes, int planes, int largest, bool nt,
+                  const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs,
+                  hipStream_t stream = nullptr);
 // one sweep phase's kernel instances each (sgm_path_first/mid/last.hip)
 int launch_path_first(hipStream_t st, int R, int sum_bytes, int mode, const PathJobs &jobs,
                       const PathArgs &A, int waves);
@@ -172,11 +189,12 @@ struct sgm_context {
   std::atomic<int> interrupt{0};
   bool last_compact = false;
   int sweeps = SGM_SWEEPS_AUTO;  // sgm_set_sweeps
-  // longest-first line orders of the plane sweeps, by buffer name: the host
-  // copy and the (w, h, matching directions, directions, first dx, dy) it is for
+  // longest-first orders of a launch's waves, by buffer name: the host copy and
+  // the (w, h, matching directions, directions, first dx, dy, lines per wave)
+  // it is for
   struct LineOrder {
     std::vector<int> host;
-    int key[6] = {0, 0, 0, 0, 0, 0};
+    int key[7] = {0, 0, 0, 0, 0, 0, 0};
   };
   std::map<std::string, LineOrder> line_orders;
   int last_sweeps = SGM_SWEEPS_SEQUENTIAL;

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 #pragma clang fp contract(off)
 
 namespace sgm {
@@ -271,6 +273,8 @@ struct CostJob {
 struct CostArgs {
   int mode, ww, wh, words, weight, adcap, gradcap, inv_code;
   int u8;  // uint8 cost volume (census-family costs <= 120, 255 = invalid 512)
+  // codes of an invalid cell and of a pad cell (k >= D) as stored in the volume
+  int inv_store, pad_store;
 };
 
 // Stores the costs of disparities k0 .. k0+3 of pixel p.
@@ -546,9 +550,10 @@ __device__ __forceinline__ void zncc_band(const CostJob &J, const CostArgs &A, i
         c = c > -1.0 ? c : -1.0;
         value = ok ? (int)round_half_up_d((1.0 - c) * .5 * bits) : 512;
       }
-      value = kin ? value : (MODE == 4 ? A.inv_code : 512);
+      if (MODE != 4) value = value == 512 ? A.inv_store : value;
+      value = kin ? value : A.pad_store;
       if (kst) {
-        if (OUT8) out[(size_t)xo * ostep] = (uint8_t)min(value, 255);
+        if (OUT8) out[(size_t)xo * ostep] = (uint8_t)value;
         else *(uint16_t *)(out + (size_t)xo * ostep) = (uint16_t)value;
       }
       if (xo + 1 < kZnccTX) {
@@ -586,7 +591,7 @@ static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArg
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int k = k0 + j;
-    int value = A.inv_code;
+    int value = k < J.D ? A.inv_store : A.pad_store;
     if (pix_ok && k < J.D) {
       const int disp = J.minD + k;
       const long long t = (long long)x + (J.reverse ? (long long)disp : -(long long)disp);
@@ -603,6 +608,7 @@ static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArg
 }  // namespace sgm
 
 #include "sgm_paths.h"
+#include "sgm_excess.h"
 
 namespace sgm {
 

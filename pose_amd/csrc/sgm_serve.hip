@@ -253,19 +253,18 @@ void sgm_server::run() {
         }
       }
       // Shrink until the group fits the pool (FIFO: keep the oldest).  Each
-      // group first tries path-cost planes, then resident cost and aggregate
+      // group first tries excess planes, then resident cost and aggregate
       // volumes, then recomputed census costs.
       size_t off = 0;
       int recompute = 0, planes = 0;
       const bool can_recompute = batch_recompute_possible(&params, ctx->keep_volumes);
-      const bool can_planes = ctx->volume_policy != SGM_VOLUME_RECOMPUTE &&
-                              batch_planes_possible(ctx, &params, SGM_BATCH_PHASED);
       while (!take.empty()) {
         std::vector<sgm_pair> prs;
         for (Request *r : take) prs.push_back(r->pair);
         const int n = (int)prs.size();
         const size_t tables = batch_table_bytes(n, &params);
-        if (can_planes) {
+        if (ctx->volume_policy != SGM_VOLUME_RECOMPUTE &&
+            batch_planes_possible(ctx, &params, prs.data(), n, SGM_BATCH_PHASED)) {
           recompute = 0;
           planes = 1;
           bytes = batch_arena_bytes(&params, prs.data(), n, 0, false, true) + tables;
@@ -398,7 +397,7 @@ void sgm_server::run() {
 // device bytes the lane will hold after serving it, plus what the other lanes
 // hold, fit the budget.  The lane's cached buffers are reused where they are
 // large enough, so that footprint counts each of the pair's buffers at the
-// larger of its cached and required size.  Plans, preferred first: path-cost
+// larger of its cached and required size.  Plans, preferred first: excess
 // planes, paired sweeps, one aggregate with the cost volume, one aggregate
 // with recomputed census costs (as the sweep schedule and the volume policy
 // allow).  Tried in order: every plan on the lane's cached buffers as they
@@ -430,10 +429,10 @@ bool sgm_server::admit_lane(Slot &s) {
   int nplan = 0;
   if (with_cv) {
     if (sweeps == SGM_SWEEPS_AUTO || sweeps == SGM_SWEEPS_PLANES) {
-      if (schedule_applies(lane, &q, SGM_SWEEPS_PLANES, true))
+      if (schedule_applies(lane, &q, w, h, SGM_SWEEPS_PLANES, true))
         plans[nplan++] = {true, SGM_SWEEPS_PLANES};
     }
-    if (sweeps != SGM_SWEEPS_SEQUENTIAL && schedule_applies(lane, &q, SGM_SWEEPS_PAIRED, true))
+    if (sweeps != SGM_SWEEPS_SEQUENTIAL && schedule_applies(lane, &q, w, h, SGM_SWEEPS_PAIRED, true))
       plans[nplan++] = {true, SGM_SWEEPS_PAIRED};
     plans[nplan++] = {true, SGM_SWEEPS_SEQUENTIAL};
   }
