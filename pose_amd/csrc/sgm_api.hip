@@ -802,6 +802,68 @@ void excess_codes(CostArgs &A) {
   A.pad_store = A.u8 ? 255 : 0x8FFF;
 }
 
+// Whether the band cost kernel (sgm_cost.h) takes the pair: a census-family
+// cost whose numerators stay below 2^31, a wave shape for the padded range, and
+// row segments of a wave within a 32-bit offset of each other.
+bool band_possible(const sgm_params *p, int w, int h) {
+  int lanes, R;
+  const int Dp = padded_disparities(p->disparities);
+  if (p->cost > SGM_COST_CENSUS_GRADIENT || !excess_shape(Dp, lanes, R) ||
+      8 * (int64_t)std::max(w, h) * Dp >= (int64_t)1 << 30)
+    return false;
+  if (p->cost == SGM_COST_CENSUS) return true;
+  const int64_t bits = p->window_w * p->window_h - 1;
+  const int64_t cap = p->cost == SGM_COST_AD_CENSUS ? p->ad_truncation : p->gradient_truncation;
+  const int64_t diff = std::min<int64_t>(cap, p->cost == SGM_COST_AD_CENSUS ? 255 : 1020);
+  return p->census_weight * bits * cap + (1000 - p->census_weight) * diff * bits + 500 * cap <
+             (int64_t)1 << 31 && 1000 * cap < (int64_t)1 << 31;
+}
+
+// Pixels per row segment for `pixels` pixels in all: long segments load their
+// first targets less often, short ones give small images enough waves (4096
+// waves are four per SIMD).
+int band_segment(const sgm_params *p, int64_t pixels) {
+  int lanes = 64, R = 0;
+  excess_shape(padded_disparities(p->disparities), lanes, R);
+  int seg = 128;
+  while (seg > 32 && pixels / seg / (64 / lanes) < 4096) seg /= 2;
+  return seg;
+}
+
+// Arguments of the band cost kernel; the caller fills in the waves.  `excess`:
+// the volume codes of the excess-plane kernels.
+BandArgs band_args(const sgm_params *p, int njobs, bool excess) {
+  BandArgs A;
+  memset(&A, 0, sizeof A);
+  A.njobs = njobs;
+  A.gradient = p->cost == SGM_COST_CENSUS_GRADIENT;
+  A.magic = 1;
+  if (p->cost != SGM_COST_CENSUS) {
+    const uint32_t bits = p->window_w * p->window_h - 1;
+    A.cap = A.gradient ? p->gradient_truncation : p->ad_truncation;
+    A.wa = p->census_weight * A.cap;
+    A.wb = (1000 - p->census_weight) * bits;
+    A.half = 1000 * A.cap / 2;
+    band_division(1000 * A.cap, A.magic, A.shift);
+  }
+  CostArgs C = cost_args(p);
+  if (excess) excess_codes(C);
+  const uint32_t rep = C.u8 ? 0x01010101u : 0x00010001u;
+  A.inv = (uint32_t)C.inv_store * rep;
+  A.pad = (uint32_t)C.pad_store * rep;
+  return A;
+}
+
+int launch_band(sgm_context *ctx, int Dp, const sgm_params *p, const PathJobs &jobs,
+                const BandArgs &A, hipStream_t stream) {
+  ProfileScope ps(ctx, "path_cost");
+  if (A.total <= 0) return SGM_OK;
+  hipStream_t st = stream ? stream : ctx->stream;
+  const bool diff = p->cost != SGM_COST_CENSUS;
+  return cost_u8(p) ? launch_band8(st, Dp, words_of(p), diff, jobs, A)
+                    : launch_band16(st, Dp, words_of(p), diff, jobs, A);
+}
+
 // Cost rows [J.y0, J.y0 + rows) of every job (rows < 0: the whole image).
 int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h, int Dp,
                 const sgm_params *p, int rows, bool force_u16, bool excess) {
@@ -887,12 +949,10 @@ int launch_path(sgm_context *ctx, int R, int sum_bytes, int mode, const PathJobs
                 const PathArgs &A, int phase, int waves, hipStream_t stream) {
   ProfileScope ps(ctx, phase == PHASE_FIRST ? "path_first"
                        : phase == PHASE_MID ? "path_mid"
-                       : phase == PHASE_COST ? "path_cost"
                                              : "path_last");
   if (A.total_lines <= 0) return SGM_OK;
   hipStream_t st = stream ? stream : ctx->stream;
   if (phase == PHASE_FIRST) return launch_path_first(st, R, sum_bytes, mode, jobs, A, waves);
-  if (phase == PHASE_COST) return launch_path_cost(st, R, sum_bytes, mode, jobs, A, waves);
   if (phase == PHASE_MID) return launch_path_mid(st, R, sum_bytes, mode, jobs, A, waves);
   return launch_path_last(st, R, sum_bytes, mode, jobs, A, waves);
 }
@@ -1938,7 +1998,8 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
   const bool nt = (mode == 4 || mode == 1) && R <= 8 &&
                   (int64_t)nd * w * h * Dp * vol_bytes > (int64_t)768 << 20;
   if (nt) mode |= MODE_NT;
-  if (!fused && !recompute) {
+  const bool band = !recompute && (B.nplanes || !fused) && band_possible(p, w, h);
+  if (!fused && !recompute && !band) {
     CostJobs cj;
     memset(&cj, 0, sizeof cj);
     for (int i = 0; i < nd; i++) {
@@ -1978,6 +2039,7 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     J.desc_a = B.desc[d];
     J.desc_b = B.desc[o];
     J.mask_b = B.mask[o];
+    J.gray_b = B.gray[o];
     J.cost_out = B.cost[d];
     J.disp = B.disp[d];
     J.reasons = d == out_slot ? reasons : nullptr;
@@ -2005,21 +2067,23 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     (void)hipStreamSynchronize(ctx->stream);
     return true;
   };
+  if (band) {
+    BandArgs A = band_args(p, nd, B.nplanes > 0);
+    int lanes = 64, er = 0;
+    excess_shape(Dp, lanes, er);
+    A.seg = band_segment(p, (int64_t)nd * w * h);
+    A.split = (h * band_segments(w, A.seg) + 64 / lanes - 1) / (64 / lanes);
+    A.total = nd * A.split;
+    if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
+    if ((rc = launch_band(ctx, Dp, p, pj, A))) return rc;
+  }
   if (B.nplanes) {
-    // Excess planes: the census cost pass (fused census cost; other costs come
-    // from the cost kernel above), every direction in one launch, each into its
-    // plane, and the winner search over the planes.
+    // Excess planes: every direction in one launch, each into its plane, and
+    // the winner search over the planes.
     ctx->last_sweeps = B.schedule;
     const int cost_bytes = cost_u8(p) ? 1 : 2;
     const bool stream = (int64_t)nd * w * h * Dp * (cost_bytes + B.nplanes) > kStreamBytes;
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
-    if (fused) {
-      PathArgs Ac = dir_args(0);
-      Ac.split = h * cost_segments(w);
-      Ac.total_lines = nd * Ac.split;
-      if ((rc = launch_path(ctx, R, sb, 2 | (stream ? MODE_NT : 0), pj, Ac, PHASE_COST, waves)))
-        return rc;
-    }
     for (int i = 0; i < nd; i++) pj.local[i].sum = B.planes[slots[i]];
     ExcessArgs E = excess_args(p, nd, B.nplanes);
     int lanes = 0, er = 0;

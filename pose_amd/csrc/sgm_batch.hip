@@ -112,7 +112,7 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     g.sub = sub;
     const int per = b->planes ? 64 / (key.second / 64) : 1;  // lines per wave
     std::vector<PathJob> gj;
-    int64_t volume = 0;
+    int64_t volume = 0, pixels = 0;
     bool aligned = true;
     for (size_t j = 0; j < jobs.size(); j++) {
       const PathJob &J = jobs[j];
@@ -121,6 +121,7 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
         volume += (int64_t)J.w * J.h * J.Dp *
                   (b->planes ? 1 + b->nplanes : b->cost8 ? 3 : 4);
         aligned &= J.Dp % 64 == 0;
+        pixels += (int64_t)J.w * J.h;
         g.Dp = J.Dp;
         g.w = std::max(g.w, J.w);
         g.h = std::max(g.h, J.h);
@@ -128,6 +129,9 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     }
     if (gj.empty()) continue;
     g.njobs = (int)gj.size();
+    sgm_params gp = b->params;
+    gp.disparities = g.Dp;
+    g.seg = band_segment(&gp, pixels);
     // stream the volumes past the caches as the plain path does: whole 64-byte
     // lines only, volumes far beyond the 256 MB MALL
     g.nt = b->planes ? volume > kStreamBytes
@@ -137,12 +141,13 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     host.resize(pd.jobs_off + gj.size() * sizeof(PathJob));
     memcpy(host.data() + pd.jobs_off, gj.data(), gj.size() * sizeof(PathJob));
     for (int cls = 0; cls < 4; cls++) {
-      // the waves of line classes 0..2, and 3: the row segments of the census
-      // cost pass
+      // the waves of line classes 0..2, and 3: the row segments of the cost pass
       std::vector<int> lb(gj.size() + 1, 0);
-      for (size_t j = 0; j < gj.size(); j++)
-        lb[j + 1] = lb[j] + (cls == 3 ? gj[j].h * cost_segments(gj[j].w)
-                                      : (lines_of(cls, gj[j].w, gj[j].h) + per - 1) / per);
+      for (size_t j = 0; j < gj.size(); j++) {
+        const int n = cls == 3 ? gj[j].h * band_segments(gj[j].w, g.seg)
+                               : lines_of(cls, gj[j].w, gj[j].h);
+        lb[j + 1] = lb[j] + (n + per - 1) / per;
+      }
       g.total_lines[cls] = lb.back();
       pd.lb_off[cls] = align_up(host.size(), 256);
       host.resize(pd.lb_off[cls] + lb.size() * sizeof(int));
@@ -277,12 +282,11 @@ static int phased_enqueue(sgm_batch *b) {
       PathJobs pj;
       memset(&pj, 0, sizeof pj);
       pj.table = g.jobs;
-      PathArgs Ac = path_args(p, 0, g.njobs, 0, 0);
-      Ac.total_lines = g.total_lines[3];
-      pj.line_begin = g.line_begin[3];  // row segments of the cost pass
-      if ((rc = launch_path(ctx, g.R, sb, 2 | (g.nt ? MODE_NT : 0), pj, Ac, PHASE_COST,
-                            path_waves(ctx, g.R), st)))
-        return rc;
+      BandArgs A = band_args(p, g.njobs, true);
+      A.seg = g.seg;
+      A.total = g.total_lines[3];
+      A.wave_begin = g.line_begin[3];
+      if ((rc = launch_band(ctx, g.Dp, p, pj, A, st))) return rc;
       ExcessArgs E = excess_args(p, g.njobs, b->nplanes);
       for (int k = 0; k < E.ndirs; k++) {
         E.begin[k] = E.total;
@@ -727,6 +731,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
       J.desc_a = (const uint64_t *)P8(o.desc[d]);
       J.desc_b = (const uint64_t *)P8(o.desc[od]);
       J.mask_b = P8(o.mask[od]);
+      J.gray_b = s.gray[od];
       J.cost_out = b->recompute ? nullptr : (uint16_t *)P8(o.cost[d]);
       J.disp = s.disp[d];
       J.reasons = d == 0 ? P8(o.rtmp) : nullptr;

@@ -78,6 +78,7 @@ struct sgm_batch {
     bool nt = false;
     const sgm::PathJob *jobs = nullptr;
     int Dp = 0, w = 0, h = 0;  // padded disparities of a job, largest sizes
+    int seg = 128;             // pixels per row segment of the cost pass
     // waves per line class (horizontal, vertical, diagonal, cost-pass row segments)
     const int *line_begin[4] = {nullptr, nullptr, nullptr, nullptr};
     int total_lines[4] = {0, 0, 0, 0};

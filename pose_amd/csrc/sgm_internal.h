@@ -133,6 +133,16 @@ int launch_check(const char *what);
 int launch_path_pair(sgm_context *ctx, int R, int mode, int phase_b, const PathJobs &ja,
                      const PathArgs &A, const PathJobs &jb, const PathArgs &B, int waves,
                      hipStream_t stream = nullptr);
+// census-family cost volumes (sgm_cost.h), on `stream` (the context's when null)
+bool band_possible(const sgm_params *p, int w, int h);
+int band_segment(const sgm_params *p, int64_t pixels);
+BandArgs band_args(const sgm_params *p, int njobs, bool excess);
+int launch_band(sgm_context *ctx, int Dp, const sgm_params *p, const PathJobs &jobs,
+                const BandArgs &A, hipStream_t stream = nullptr);
+int launch_band8(hipStream_t st, int Dp, int words, bool diff, const PathJobs &jobs,
+                 const BandArgs &A);
+int launch_band16(hipStream_t st, int Dp, int words, bool diff, const PathJobs &jobs,
+                  const BandArgs &A);
 // every direction of `A`, each storing its excess plane (sgm_excess.h)
 int launch_excess(sgm_context *ctx, int Dp, int cost_bytes, bool nt, const PathJobs &jobs,
                   const ExcessArgs &A, hipStream_t stream = nullptr);
@@ -147,8 +157,6 @@ int launch_path_first(hipStream_t st, int R, int sum_bytes, int mode, const Path
 int launch_path_mid(hipStream_t st, int R, int sum_bytes, int mode, const PathJobs &jobs,
                     const PathArgs &A, int waves);
 int launch_path_last(hipStream_t st, int R, int sum_bytes, int mode, const PathJobs &jobs,
-                     const PathArgs &A, int waves);
-int launch_path_cost(hipStream_t st, int R, int sum_bytes, int mode, const PathJobs &jobs,
                      const PathArgs &A, int waves);
 int path_lanes(const sgm_params *p);
 bool fused_cost(const sgm_params *p);

@@ -609,6 +609,7 @@ static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArg
 
 #include "sgm_paths.h"
 #include "sgm_excess.h"
+#include "sgm_cost.h"
 
 namespace sgm {
 

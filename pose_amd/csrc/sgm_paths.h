@@ -40,6 +40,7 @@ struct PathJob {
   // fused first sweep (census cost computed on the fly, written to cost_out)
   const uint64_t *desc_a, *desc_b;
   const uint8_t *mask_b;
+  const uint8_t *gray_b;    // target image
   uint16_t *cost_out;
   // last sweep outputs
   float *disp;
@@ -66,14 +67,7 @@ struct PathArgs {
   const int *order;
 };
 
-// Row segment of the census cost pass: one wave per kCostSegment pixels of a
-// row, so the pass runs many more waves than rows.
-constexpr int kCostSegment = 128;
-__host__ __device__ inline int cost_segments(int w) { return (w + kCostSegment - 1) / kCostSegment; }
-
-// PHASE_COST: the fused census cost of a left-to-right line, written to the
-// cost volume, with no path recurrence (the cost pass of the plane schedule).
-enum { PHASE_FIRST = 0, PHASE_MID = 1, PHASE_LAST = 2, PHASE_COST = 3 };
+enum { PHASE_FIRST = 0, PHASE_MID = 1, PHASE_LAST = 2 };
 
 // Selection code bits (one byte per pixel, counted by the L-R / count kernels).
 enum { CODE_SELECTED = 1, CODE_BOUNDARY = 2, CODE_AMBIGUOUS = 3, CODE_FULL = 4, CODE_LOWER = 8,
@@ -827,23 +821,6 @@ __device__ __forceinline__ void census_costs(const uint64_t *tw, uint32_t alo, u
   for (int i = 0; i < R / 2; i++) c[i] = (uint32_t)cv[2 * i] | ((uint32_t)cv[2 * i + 1] << 16);
 }
 
-// The same with the codes of the excess-plane schedule (sgm_excess.h): 254 for
-// an invalid cell, 255 for a pad cell.
-template <int R>
-__device__ __forceinline__ void census_codes(const uint64_t *tw, uint32_t alo, uint32_t ahi,
-                                             bool ok, int kbase, int D, uint32_t *c) {
-  int cv[R];
-#pragma unroll
-  for (int j = 0; j < R; j++) {
-    const uint32_t wl = (uint32_t)tw[j], wh = (uint32_t)(tw[j] >> 32);
-    const int ham = __builtin_popcount(wl ^ alo) + __builtin_popcount((wh ^ ahi) & 0x7FFFFFFFu);
-    const bool in = kbase + j < D;
-    cv[j] = (ok && (wh >> 31) && in) ? ham : in ? 254 : 255;
-  }
-#pragma unroll
-  for (int i = 0; i < R / 2; i++) c[i] = (uint32_t)cv[2 * i] | ((uint32_t)cv[2 * i + 1] << 16);
-}
-
 // SLIDE_UP: direction of the sliding target window of a horizontal computed-cost
 // line, fixed at compile time (1: towards higher x indices of the window, 0:
 // lower) so the window rotates by register renaming in the unrolled steps; -1
@@ -858,8 +835,6 @@ struct PkSweep {
   static constexpr bool kLoaded = CM == CM_LOAD || CM == CM_LOAD8;
   static constexpr int NC = CM == CM_LOAD8 ? (R + 3) / 4 : NP;  // dwords of loaded cost per slot
   static constexpr int kDirect = CM == CM_RECOMPUTE ? PF : 1;  // direct target-row prefetch slots
-  static_assert(PHASE != PHASE_COST || CM == CM_FUSED, "the cost pass computes the census cost");
-
   const PathJob &J;
   const PathArgs &A;
   const int *p2_table;
@@ -900,13 +875,6 @@ struct PkSweep {
     sloff = kbase < J.Dp ? kbase * 2 : kOutOfRange;
     sboff = kbase < J.Dp ? kbase : kOutOfRange;
     line_start(line, A.dx, A.dy, J.w, J.h, x0, y0, len);
-    if constexpr (PHASE == PHASE_COST) {
-      // a left-to-right row segment: line = row * segments + segment
-      const int nseg = cost_segments(J.w);
-      y0 = line / nseg;
-      x0 = (line - y0 * nseg) * kCostSegment;
-      len = min(kCostSegment, J.w - x0);
-    }
     step_off = (ptrdiff_t)A.dy * J.w + A.dx;
     p0 = (ptrdiff_t)y0 * J.w + x0;
     row_bytes = (uint32_t)J.Dp * 2u;
@@ -1047,10 +1015,7 @@ struct PkSweep {
       const uint32_t ahi = (uint32_t)__builtin_amdgcn_readlane((int)meta.da_hi, ml);
       const bool ok = __builtin_amdgcn_readlane(meta.ok, ml) != 0;
       if (slide) {
-        if constexpr (PHASE == PHASE_COST)
-          census_codes<R>(win, alo, ahi, ok, kbase, J.D, c);
-        else
-          census_costs<R>(win, alo, ahi, ok, kbase, J.D, A.inv_code, c);
+        census_costs<R>(win, alo, ahi, ok, kbase, J.D, A.inv_code, c);
         const uint32_t elo = (uint32_t)__builtin_amdgcn_readlane((int)meta.e_lo, ml);
         const uint32_t ehi = (uint32_t)__builtin_amdgcn_readlane((int)meta.e_hi, ml);
         slide_window(elo, ehi);
@@ -1064,7 +1029,6 @@ struct PkSweep {
         bstore_bytes<R, POL>(raw, make_rsrc(st_c, cost_row_bytes), sboff);
         st_c += cstep;
       }
-      if constexpr (PHASE == PHASE_COST) return;  // the cost pass: no recurrence
     } else if constexpr (CM == CM_LOAD8) {
       widen_costs<NP>(cb[slot], c);
     } else {
