@@ -28,6 +28,7 @@
 #include "sgm_filters.h"
 #include "sgm_strips.h"
 #include "sgm_compact.h"
+#include "sgm_compact_lines.h"
 
 using namespace sgm;
 
@@ -1622,6 +1623,15 @@ int run_directions_streamed(sgm_context *ctx, const sgm_params *p, int w, int h,
   return SGM_OK;
 }
 
+}  // namespace
+
+namespace sgm {
+int launch_compact_lines(sgm_context *ctx, int lanes, int R, int phase, const CompactJobs &J,
+                         const CompactLineArgs &A);
+}
+
+namespace {
+
 template <int R, int PH, bool HREC>
 void launch_compact_t(sgm_context *ctx, const CompactJobs &J, const PathArgs &A,
                       const CompactArgs &E, int Dp) {
@@ -1793,6 +1803,7 @@ int run_directions_esgm(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
     K.cost = Cj.cost;
     K.mask = B.mask[d];
     K.gray = B.gray[d];
+    K.gm = B.gm[d];
     K.cand = B.e_cand + i * n * C;
     K.sums = B.e_sums + i * n * 3 * C;
     K.outside = B.e_outside + i * n;
@@ -1842,7 +1853,46 @@ int run_directions_esgm(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
     (void)hipStreamSynchronize(ctx->stream);
     return true;
   };
+  // whole-image line sweeps, several lines per wave (sgm_compact_lines.h): lanes
+  // of 8 disparities (4 at 64), the fewest lanes that hold the range.  16 per
+  // lane and half the lanes is no faster where directions run together (a wave
+  // instruction more per cell against fewer registers and more waves) and 13%
+  // slower in the sum pass, whose launches of one direction leave SIMDs idle.
+  const bool lined = computed && effective_p2(p) <= kCompactLineP2 && std::max(w, h) < 65535 &&
+                     n < ((size_t)1 << 28);
+  const int lR = Dp == 64 ? 4 : 8, ln = Dp <= 128 ? 16 : Dp <= 256 ? 32 : 64;
+  for (int i = 0; i < 2; i++) sj.job[i].vr = lined ? lR : 0;
+  auto sweep_lines = [&](int phase) -> int {
+    // the sum pass accumulates: one direction per launch; the others run every
+    // direction in one
+    const bool apart = phase == ESGM_SUMS;
+    for (int d0 = 0; d0 < (apart ? p->directions : 1); d0++) {
+      if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
+      CompactLineArgs A;
+      memset(&A, 0, sizeof A);
+      A.ndirs = apart ? 1 : p->directions;
+      A.njobs = nd;
+      A.p1 = p->p1;
+      A.p2 = effective_p2(p);
+      A.edge = p->edge_scale;
+      A.C = C;
+      A.pool = pool;
+      A.first = d0 == 0;
+      for (int k = 0; k < A.ndirs; k++) {
+        const PathArgs P = path_args(p, d0 + k, nd, 0, 0);
+        A.dx[k] = P.dx;
+        A.dy[k] = P.dy;
+        A.index[k] = d0 + k;
+        A.split[k] = (lines_of(P.cls, w, h) + 64 / ln - 1) / (64 / ln);
+        A.begin[k] = A.total;
+        A.total += nd * A.split[k];
+      }
+      if (int rc2 = launch_compact_lines(ctx, ln, lR, phase, kj, A)) return rc2;
+    }
+    return SGM_OK;
+  };
   auto sweep = [&](int phase) -> int {
+    if (lined) return sweep_lines(phase);
     if (computed) {
       for (int dir = 0; dir < p->directions; dir++) {
         if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
@@ -1900,9 +1950,12 @@ int run_directions_esgm(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
     }
     return SGM_OK;
   };
-  // every proposal entry is written by the proposal sweeps; sums and bounds accumulate
-  if ((rc = launch_fill_u8(ctx, (uint8_t *)B.e_sums, 0, (size_t)nd * n * 3 * C * 2))) return rc;
-  if ((rc = launch_fill_u8(ctx, (uint8_t *)B.e_outside, 0, (size_t)nd * n * 2))) return rc;
+  // every proposal entry is written by the proposal sweeps; sums and bounds
+  // accumulate (the line sweeps' first direction stores them)
+  if (!lined) {
+    if ((rc = launch_fill_u8(ctx, (uint8_t *)B.e_sums, 0, (size_t)nd * n * 3 * C * 2))) return rc;
+    if ((rc = launch_fill_u8(ctx, (uint8_t *)B.e_outside, 0, (size_t)nd * n * 2))) return rc;
+  }
   if ((rc = launch_fill_u8(ctx, (uint8_t *)B.e_count, 0, 8))) return rc;
   if ((rc = sweep(ESGM_CANDIDATES))) return rc;
   if ((rc = sweep(ESGM_SUMS))) return rc;

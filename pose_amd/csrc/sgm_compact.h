@@ -15,7 +15,8 @@
 // selected map, reasons and counters are therefore those of ordinary SGM.
 //
 // With 1-word census windows and R <= 8 every path sweeps the whole image and
-// computes its census costs on the fly from the descriptors (HREC): no cost
+// computes its census costs on the fly from the descriptors (several lines per
+// wave in sgm_compact_lines.h; HREC here for what those do not take): no cost
 // volume at all.  Otherwise sweeps run over horizontal strips with int32 path
 // carries at the seams (sgm_strips.h), so the device holds one strip's cost
 // volume at a time: a top-down pass over the strips runs the paths with
@@ -33,6 +34,7 @@ struct CompactJob {
   const uint16_t *cost;      // strip cost volume (uint16, 512 = invalid), [(y - y0) * w + x][Dp]
   const uint8_t *mask;       // texture & valid of the reference image (whole image)
   const uint8_t *gray;       // reference image (whole image)
+  const uint16_t *gm;        // gray | mask << 8 of the reference image
   const int *carry_in;       // [x][Dp] path value before the strip, or nullptr
   int *carry_out;            // [x][Dp] path value at the strip's exit row, or nullptr
   uint16_t *cand;            // [p][C] proposals, path r at [r * pool, r * pool + pool); 65535 = none
@@ -363,6 +365,7 @@ struct SummaryJob {
   int *pixels;                     // [slot] pixel
   int *count;                      // verification slots handed out
   const uint16_t *verify;          // [slot - lo][Dp] (verification winners)
+  int vr;                          // disparities per lane of its rows (verify_cell; 0: in order)
   int lo, hi;
   int w, h, D, Dp, minD, rx, ry, reverse;
 };
@@ -399,36 +402,56 @@ __device__ __forceinline__ void put_summary(uint32_t *out, int best, int flags, 
 
 // Winner over the proposals (esgm_select, GpuCandidateStereo.java:456-478) and
 // the certification of GpuCandidateStereo.java:82-102; pixels that are not
-// certified get a verification slot.  One thread per pixel.
-__global__ __launch_bounds__(256) void esgm_summary_kernel(SummaryJobs jobs, int C, double uniq) {
+// certified get a verification slot.  One thread per pixel, four proposals to a
+// load, the target test only for sums that could matter: 1600x1067, two proposals
+// per path and eight paths 1.28 -> 0.28 ms (16-bit loads, a test per proposal).
+static __global__ __launch_bounds__(256) void esgm_summary_kernel(SummaryJobs jobs, int C, double uniq) {
   const SummaryJob J = jobs.job[blockIdx.y];
   const size_t n = (size_t)J.w * J.h;
   const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
   bool unresolved = false;
   if (p < n) {
     const int x = (int)(p % J.w), y = (int)(p / J.w);
-    const uint16_t *cand = J.cand + p * C, *sums = J.sums + p * (size_t)(3 * C);
-    int best = -1, value = 0x7FFFFFFF, second = 0x7FFFFFFF, before = -1, after = -1, owner = -1;
-    for (int j = 0; j < C; j++) {
-      const int k = cand[j], v = sums[3 * j + 1];
-      if (k < J.D && (v < value || (v == value && (best < 0 || k < best)))) {
-        best = k;
-        value = v;
-        owner = j;
-      }
+    // four proposals at a time (their number is a multiple of 4: 8-byte loads)
+    const uint2 *cand = (const uint2 *)(J.cand + p * C);
+    const uint2 *sums = (const uint2 *)(J.sums + p * (size_t)(3 * C));
+    int best = -1, value = 0x7FFFFFFF, second = 0x7FFFFFFF, before = -1, after = -1;
+    int left = 0, right = 0;  // of the best so far
+    auto four = [&](int j, int *k, int (*v)[3]) {
+      const uint2 c = cand[j], a = sums[3 * j], b = sums[3 * j + 1], d = sums[3 * j + 2];
+      const uint32_t in[2] = {c.x, c.y}, s[6] = {a.x, a.y, b.x, b.y, d.x, d.y};
+#pragma unroll
+      for (int i = 0; i < 4; i++) k[i] = (int)(in[i / 2] >> (i % 2 * 16) & 0xFFFF);
+#pragma unroll
+      for (int i = 0; i < 12; i++) v[i / 3][i % 3] = (int)(s[i / 2] >> (i % 2 * 16) & 0xFFFF);
+    };
+    for (int j = 0; j < C / 4; j++) {
+      int k[4], v[4][3];
+      four(j, k, v);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (k[i] < J.D && (v[i][1] < value || (v[i][1] == value && (best < 0 || k[i] < best)))) {
+          best = k[i];
+          value = v[i][1];
+          left = v[i][0];
+          right = v[i][2];
+        }
     }
     const bool pix = esgm_pixel_ok(J, x, y);
-    if (owner >= 0 && pix) {
-      if (esgm_target_ok(J, x, y, best - 1)) before = sums[3 * owner];
-      if (esgm_target_ok(J, x, y, best + 1)) after = sums[3 * owner + 2];
-      for (int j = 0; j < C; j++) {
-        const int kc = (int)cand[j];
+    if (best >= 0 && pix) {
+      if (esgm_target_ok(J, x, y, best - 1)) before = left;
+      if (esgm_target_ok(J, x, y, best + 1)) after = right;
+      for (int j = 0; j < C / 4; j++) {
+        int k[4], v[4][3];
+        four(j, k, v);
 #pragma unroll
-        for (int o = 0; o < 3; o++) {
-          const int k = kc + o - 1;
-          if (abs(k - best) > 1 && esgm_target_ok(J, x, y, k))
-            second = min(second, (int)sums[3 * j + o]);
-        }
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int o = 0; o < 3; o++) {
+            const int kk = k[i] + o - 1;
+            if (v[i][o] < second && abs(kk - best) > 1 && esgm_target_ok(J, x, y, kk))
+              second = v[i][o];
+          }
       }
     }
     const int flags = pix ? (esgm_target_ok(J, x, y, 0) ? 1 : 0) |
@@ -463,6 +486,15 @@ __global__ __launch_bounds__(256) void esgm_summary_kernel(SummaryJobs jobs, int
   }
 }
 
+// Position of disparity k in a verified pixel's row of Dp cells: in order, or as
+// the line sweeps add it up, lanes of vr disparities with the packed pairs
+// (0, 2), (1, 3), (4, 6), ... of all lanes side by side, in ascending columns.
+__device__ __forceinline__ int verify_cell(int k, int vr, int Dp, int reverse) {
+  if (!vr) return k;
+  const int l = k / vr, j = reverse ? k - l * vr : vr - 1 - (k - l * vr);
+  return (((j >> 2) * 2 + (j & 1)) * (Dp / vr) + l) * 2 + ((j >> 1) & 1);
+}
+
 // Exact winners of the verified pixels of one group (slots [lo, hi)): one wave
 // per pixel over its full aggregate vector.
 template <int R>
@@ -480,7 +512,7 @@ __global__ __launch_bounds__(256) void esgm_verify_kernel(SummaryJobs jobs) {
   for (int j = 0; j < R; j++) {
     const int k = kbase + j;
     valid[j] = esgm_valid(J, x, y, k) ? 1 : 0;
-    S[j] = k < J.D ? (int)row[k] : 0x7FFFFFFF;
+    S[j] = k < J.D ? (int)row[verify_cell(k, J.vr, J.Dp, J.reverse)] : 0x7FFFFFFF;
   }
   const Winner win = wta_reduce<R, false>(S, valid, kbase, J.D);
   if (lane_id() == 0)
@@ -499,7 +531,7 @@ struct SelectJobs {
   SelectJob job[2];
 };
 
-__global__ __launch_bounds__(256) void esgm_select_kernel(SelectJobs jobs, PathArgs A) {
+static __global__ __launch_bounds__(256) void esgm_select_kernel(SelectJobs jobs, PathArgs A) {
   const SelectJob &S = jobs.job[blockIdx.z];
   const int waves = blockDim.x >> 6;
   const int chunk = __builtin_amdgcn_readfirstlane((int)blockIdx.x * waves + (int)(threadIdx.x >> 6));
