@@ -799,7 +799,7 @@ CostArgs cost_args(const sgm_params *p) {
 
 // Volume codes of the excess-plane kernels (sgm_excess.h).
 void excess_codes(CostArgs &A) {
-  A.inv_store = A.u8 ? 254 : A.inv_code;
+  A.inv_store = A.u8 ? 254 : 0x8000 | A.inv_code;
   A.pad_store = A.u8 ? 255 : 0x8FFF;
 }
 
@@ -1074,7 +1074,7 @@ int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule) {
 bool sgm::excess_possible(const sgm_params *p, int w, int h) {
   int lanes, R;
   const int Dp = padded_disparities(p->disparities);
-  return aggregate_bytes(p) == 2 && effective_p2(p) <= 255 && excess_shape(Dp, lanes, R) &&
+  return effective_p2(p) <= 255 && excess_shape(Dp, lanes, R) &&
          4 * (int64_t)std::max(w, h) * Dp * kMaxExcessDirs < (int64_t)1 << 30;
 }
 
@@ -1104,14 +1104,21 @@ int sgm::excess_plane_count(const sgm_params *p, int64_t cells) {
 
 // Excess planes per pixel of a pair on the resident plan under `schedule` (0:
 // aggregate volumes).  With 4 paths the two partial aggregates of the paired
-// schedule are the room of one plane per path.
-int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule) {
+// schedule are the room of one plane per path.  A 32-bit aggregate is the room
+// of four planes of its own, one per path or per pair of opposite paths where
+// two excesses fit a byte: path costs and aggregates stay 32-bit (WideState,
+// winner32_kernel), but no aggregate goes through memory, and 19 + 8 bytes a
+// cell replace 74 of eight sequential sweeps.
+int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
+                       bool cost_volume) {
   if (schedule == SGM_SWEEPS_PLANES)
     return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities));
-  if (schedule == SGM_SWEEPS_PAIRED && p->directions == 4 && !ctx->keep_volumes &&
-      excess_possible(p, w, h))
-    return 4;
-  return 0;
+  if (ctx->keep_volumes || !cost_volume || !excess_possible(p, w, h)) return 0;
+  if (schedule == SGM_SWEEPS_PAIRED) return p->directions == 4 ? 4 : 0;
+  return aggregate_bytes(p) == 4 && ctx->sweeps != SGM_SWEEPS_SEQUENTIAL &&
+                 (p->directions == 4 || 2 * effective_p2(p) <= 255)
+             ? 4
+             : 0;
 }
 
 // Sweep schedule of a resident pair under `budget` (SGM_SWEEPS_SEQUENTIAL,
@@ -1183,7 +1190,7 @@ static std::vector<std::pair<std::string, size_t>> pair_buffer_list(const sgm_pa
 int64_t sgm::resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h,
                                 bool cost_volume, int schedule, bool fresh) {
   int64_t total = fresh ? 0 : ctx->allocated;
-  const int planes = excess_planes(ctx, p, w, h, schedule);
+  const int planes = excess_planes(ctx, p, w, h, schedule, cost_volume);
   for (const auto &b : pair_buffer_list(p, w, h, true, cost_volume, schedule, planes)) {
     if (fresh) {
       total += (int64_t)b.second;
@@ -1208,7 +1215,7 @@ int ensure_pair_buffers(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
   const bool recompute = !rows && recompute_cost(ctx, p, w, h);
   const int schedule =
       rows ? SGM_SWEEPS_SEQUENTIAL : sweep_schedule(ctx, p, w, h, !recompute, ctx->budget);
-  const int planes = excess_planes(ctx, p, w, h, schedule);
+  const int planes = rows ? 0 : excess_planes(ctx, p, w, h, schedule, !recompute);
   int rc;
 #define ENSURE(name, bytes)                                                   \
   if ((rc = ctx->buffers[name].ensure(ctx, (bytes), name)) != SGM_OK) return rc;
@@ -2155,8 +2162,14 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     E.order = line_order(ctx, "excess_order", E.ndirs, E.dx, E.dy, E.split, E.begin, E.total, w, h,
                          nd, per);
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
-    if ((rc = launch_excess(ctx, Dp, cost_bytes, stream, pj, E))) return rc;
+    const bool wide = aggregate_bytes(p) == 4;
+    if ((rc = wide ? launch_excess32(ctx, Dp, stream, pj, E)
+                   : launch_excess(ctx, Dp, cost_bytes, stream, pj, E)))
+      return rc;
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
+    if (wide)
+      return launch_winner32(ctx, Dp, stream, pj, WinnerArgs{p->directions, p->uniqueness}, w, h,
+                             nd);
     return launch_winner(ctx, Dp, cost_bytes, B.nplanes, E.pairs ? 2 * E.p2 : E.p2, stream, pj,
                          WinnerArgs{p->directions, p->uniqueness}, w, h, nd);
   }

@@ -7,8 +7,8 @@ template <int LANES, int R, int CB, bool PAIR>
 static int launch_excess_t(hipStream_t st, bool nt, const PathJobs &jobs, const ExcessArgs &A) {
   constexpr int waves = 4;
   const unsigned blocks = (unsigned)((A.total + waves - 1) / waves);
-  if (nt) excess_kernel<LANES, R, CB, PAIR, true><<<blocks, waves * 64, 0, st>>>(jobs, A);
-  else excess_kernel<LANES, R, CB, PAIR, false><<<blocks, waves * 64, 0, st>>>(jobs, A);
+  if (nt) excess_kernel<LANES, R, CB, PAIR, true, false><<<blocks, waves * 64, 0, st>>>(jobs, A);
+  else excess_kernel<LANES, R, CB, PAIR, false, false><<<blocks, waves * 64, 0, st>>>(jobs, A);
   return launch_check("excess sweep kernel");
 }
 

@@ -68,7 +68,8 @@ int64_t resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h, 
                            int schedule, bool fresh);
 bool excess_possible(const sgm_params *p, int w, int h);
 int excess_plane_count(const sgm_params *p, int64_t cells);
-int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule);
+int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
+                  bool cost_volume);
 bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                       bool cost_volume);
 int64_t schedule_bytes(const sgm_params *p, int w, int h, int schedule);
@@ -151,6 +152,10 @@ int launch_excess(sgm_context *ctx, int Dp, int cost_bytes, bool nt, const PathJ
 int launch_winner(sgm_context *ctx, int Dp, int cost_bytes, int planes, int largest, bool nt,
                   const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs,
                   hipStream_t stream = nullptr);
+// both for uint16 costs and four planes, in 32 bits
+int launch_excess32(sgm_context *ctx, int Dp, bool nt, const PathJobs &jobs, const ExcessArgs &A);
+int launch_winner32(sgm_context *ctx, int Dp, bool nt, const PathJobs &jobs, const WinnerArgs &A,
+                    int w, int h, int njobs);
 // one sweep phase's kernel instances each (sgm_path_first/mid/last.hip)
 int launch_path_first(hipStream_t st, int R, int sum_bytes, int mode, const PathJobs &jobs,
                       const PathArgs &A, int waves);
