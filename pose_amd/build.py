@@ -4,11 +4,11 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["csrc/sgm_api.hip", "csrc/sgm_path_first.hip", "csrc/sgm_path_mid.hip",
-           "csrc/sgm_path_last.hip", "csrc/sgm_path_pair.hip", "csrc/sgm_excess.hip", "csrc/sgm_excess32.hip",
-           "csrc/sgm_winner.hip", "csrc/sgm_cost8.hip", "csrc/sgm_cost16.hip",
-           "csrc/sgm_compact.hip", "csrc/sgm_batch.hip",
-           "csrc/sgm_serve.hip"]
+SOURCES = ["csrc/sgm_api.hip", "csrc/sgm_census.hip", "csrc/sgm_path_first.hip",
+           "csrc/sgm_path_mid.hip", "csrc/sgm_path_last.hip", "csrc/sgm_path_pair.hip",
+           "csrc/sgm_excess.hip", "csrc/sgm_excess32.hip", "csrc/sgm_winner.hip",
+           "csrc/sgm_cost8.hip", "csrc/sgm_cost16.hip", "csrc/sgm_compact.hip",
+           "csrc/sgm_batch.hip", "csrc/sgm_serve.hip"]
 OUTPUT = os.path.join(HERE, "libsgm_hip.so")
 
 HIPCC_FLAGS = [

@@ -770,18 +770,6 @@ int launch_fill_u64(sgm_context *ctx, unsigned long long *p, unsigned long long 
   return launch_check("fill kernel");
 }
 
-int launch_census(sgm_context *ctx, const CensusJobs &jobs, int njobs, int w, int h,
-                  const sgm_params *p) {
-  ProfileScope ps(ctx, "census");
-  dim3 grid((w + kCensusTx - 1) / kCensusTx, (h + kCensusTy - 1) / kCensusTy, njobs);
-  dim3 block(kCensusTx, kCensusTy);
-  if (words_of(p) == 1)
-    census_kernel<1><<<grid, block, 0, ctx->stream>>>(jobs, p->window_w, p->window_h);
-  else
-    census_kernel<2><<<grid, block, 0, ctx->stream>>>(jobs, p->window_w, p->window_h);
-  return launch_check("census kernel");
-}
-
 CostArgs cost_args(const sgm_params *p) {
   CostArgs A;
   A.mode = p->cost;

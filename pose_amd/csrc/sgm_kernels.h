@@ -92,7 +92,7 @@ __device__ __forceinline__ unsigned wave_min_u(unsigned u) {
 }
 
 // ---------------------------------------------------------------------------
-// Census transform + texture mask (CensusSgm.java:523-555), rectangular window.
+// Census transform + texture mask (CensusSgm.java:523-555; sgm_census.hip).
 struct CensusJob {
   const uint8_t *gray;      // input raster
   const uint8_t *valid;     // optional validity mask (0 = invalid)
@@ -115,63 +115,6 @@ constexpr int kCensusTx = 32, kCensusTy = 8;
 struct CensusJobs {
   CensusJob job[2];
 };
-
-template <int WORDS>
-__global__ __launch_bounds__(256) void census_kernel(CensusJobs jobs, int ww, int wh) {
-  const CensusJob J = jobs.job[blockIdx.z];
-  const int rx = ww >> 1, ry = wh >> 1;
-  const int x0 = blockIdx.x * kCensusTx, y0 = blockIdx.y * kCensusTy;
-  if (x0 >= J.w || y0 >= J.h) return;
-  __shared__ uint8_t tile[kCensusTy + 10][kCensusTx + 10 + 2];
-  const int tw = kCensusTx + 2 * rx, th = kCensusTy + 2 * ry;
-  const int tid = threadIdx.y * kCensusTx + threadIdx.x;
-  for (int i = tid; i < tw * th; i += 256) {
-    int ty = i / tw, tx = i - ty * tw;
-    int gx = x0 - rx + tx, gy = y0 - ry + ty;
-    tile[ty][tx] = (gx >= 0 && gx < J.w && gy >= 0 && gy < J.h) ? J.gray[(size_t)gy * J.w + gx] : 0;
-  }
-  __syncthreads();
-  const int x = x0 + threadIdx.x, y = y0 + threadIdx.y;
-  if (x >= J.w || y >= J.h) return;
-  const size_t n = (size_t)J.w * J.h, p = (size_t)y * J.w + x;
-  if (J.reasons) J.reasons[p] = 1;
-  if (J.boundary) J.boundary[p] = 0;
-  if (J.stats && p < 16) J.stats[p] = 0ULL;
-  if (J.gray_copy) J.gray_copy[p] = tile[threadIdx.y + ry][threadIdx.x + rx];
-  const bool interior = x >= rx && x < J.w - rx && y >= ry && y < J.h - ry;
-  uint64_t d0 = 0, d1 = 0;
-  int lo = 255, hi = 0, s1 = 0, s2 = 0;
-  if (interior) {
-    const int c = tile[threadIdx.y + ry][threadIdx.x + rx];
-    int bit = 0;
-    for (int yy = 0; yy < wh; yy++)
-      for (int xx = 0; xx < ww; xx++) {
-        const int v = tile[threadIdx.y + yy][threadIdx.x + xx];
-        lo = min(lo, v);
-        hi = max(hi, v);
-        s1 += v;
-        s2 += v * v;
-        if (yy == ry && xx == rx) continue;
-        const uint64_t m = (uint64_t)(v < c) << (bit & 63);
-        if (WORDS == 1 || bit < 64) d0 |= m;
-        else d1 |= m;
-        bit++;
-      }
-  }
-  uint8_t m;
-  if (J.mask_in) m = J.mask_in[p] != 0;
-  else m = interior && (hi - lo) >= 4 && (J.valid == nullptr || J.valid[p] != 0);
-  // One-word descriptors use at most 62 bits; bit 63 carries texture&valid so a
-  // sweep can test a target's usability from its descriptor alone.
-  J.desc[p] = WORDS == 1 ? (d0 | ((uint64_t)m << 63)) : d0;
-  if (WORDS > 1) J.desc[n + p] = d1;
-  J.mask[p] = m;
-  if (J.gm) J.gm[p] = (uint16_t)(tile[threadIdx.y + ry][threadIdx.x + rx] | (m << 8));
-  if (J.wsum) {
-    J.wsum[p] = s1;
-    J.wsum2[p] = s2;
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Colour-distance census (CensusSgm.colorCensus, CensusSgm.java:302-332) from
