@@ -2277,8 +2277,15 @@ int run_pair(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuffers &B
       G.reverse = d;
       G.correlation = B.refine->correlation;
       ProfileScope ps(ctx, "refine");
-      refine_kernel<<<dim3((unsigned)((w + 255) / 256), (unsigned)h), 256, 0, ctx->stream>>>(
-          orig, B.disp[d], B.gray[d], B.gray[1 - d], G);
+      const dim3 grid((unsigned)((w + 255) / 256), (unsigned)h);
+      auto run = [&](auto kernel) {
+        kernel<<<grid, 256, 0, ctx->stream>>>(orig, B.disp[d], B.gray[d], B.gray[1 - d], G);
+      };
+      if (G.r == 1) run(refine_kernel<1>);
+      else if (G.r == 2) run(refine_kernel<2>);
+      else if (G.r == 3) run(refine_kernel<3>);
+      else if (G.r == 4) run(refine_kernel<4>);
+      else run(refine_kernel<0>);
       if ((rc = launch_check("refinement kernel"))) return rc;
     }
   }
@@ -2480,17 +2487,31 @@ int run_filters(sgm_context *ctx, const sgm_params *p, const sgm_filter_params *
     if ((rc = launch_check("median kernel"))) return rc;
     work = fmed;
   }
-  photo_kernel<<<blocks, 256, 0, ctx->stream>>>(work, B.disp[1], B.bgr[0] ? B.bgr[0] : B.gray[0],
-                                                B.bgr[1] ? B.bgr[1] : B.gray[1],
-                                                B.reasons_out, B.stats, F);
+  {
+    // radii 1..4 (windows of 3 to 9 pixels) have their own instances
+    const uint8_t *l = B.bgr[0] ? B.bgr[0] : B.gray[0], *r = B.bgr[1] ? B.bgr[1] : B.gray[1];
+    auto run = [&](auto kernel) {
+      kernel<<<blocks, 256, 0, ctx->stream>>>(work, B.disp[1], l, r, B.reasons_out, B.stats, F);
+    };
+    if (F.corr_r < 1 || F.corr_r > 4) run(photo_kernel<0, 0>);
+#define RADIUS(R)                                       \
+  else if (F.corr_r == R) {                             \
+    if (F.channels == 1) run(photo_kernel<R, 1>);       \
+    else run(photo_kernel<R, 3>);                       \
+  }
+    RADIUS(1) RADIUS(2) RADIUS(3) RADIUS(4)
+#undef RADIUS
+  }
   if ((rc = launch_check("photometric kernel"))) return rc;
   if (f->speckle_size > 1) {
     const dim3 tiles((w + kCcTx - 1) / kCcTx, (h + kCcTy - 1) / kCcTy), tile(kCcTx, kCcTy);
     cc_local_kernel<<<tiles, tile, 0, ctx->stream>>>(work, parent, size, error, F);
     cc_border_kernel<<<tiles, tile, 0, ctx->stream>>>(work, parent, error, F);
-    cc_flatten_kernel<<<blocks, 256, 0, ctx->stream>>>(parent, error, n);
-    cc_size_kernel<<<blocks, 256, 0, ctx->stream>>>(parent, size, n);
-    cc_remove_kernel<<<blocks, 256, 0, ctx->stream>>>(work, parent, size, B.reasons_out, B.stats, F);
+    const size_t per = 4 * 64 * kCcChunks;
+    cc_flatten_kernel<<<(unsigned)((n + per - 1) / per), 256, 0, ctx->stream>>>(parent, size, error,
+                                                                                n);
+    const unsigned few = std::max(std::min(blocks, 256u), std::min((blocks + 3) / 4, 1024u));
+    cc_remove_kernel<<<few, 256, 0, ctx->stream>>>(work, parent, size, B.reasons_out, B.stats, F);
     if ((rc = launch_check("speckle kernels"))) return rc;
   } else {
     count_valid_kernel<<<blocks, 256, 0, ctx->stream>>>(work, B.stats, n);
