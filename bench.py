@@ -62,7 +62,8 @@ def algorithmic_bytes_per_step(w, h, D, paths):
 # Sources whose change invalidates the committed HBM traffic measurement of the
 # path sweeps (profiles/path_traffic.json carries the hash it was measured at).
 TRAFFIC_SOURCES = ["pose_amd/csrc/sgm_paths.h", "pose_amd/csrc/sgm_kernels.h",
-                   "pose_amd/csrc/sgm_excess.h", "pose_amd/csrc/sgm_path_launch.h"]
+                   "pose_amd/csrc/sgm_excess.h", "pose_amd/csrc/sgm_cost.h",
+                   "pose_amd/csrc/sgm_path_launch.h"]
 
 
 def kernel_source_hash():
@@ -402,7 +403,7 @@ def run_aggregate32(sgm, W, H, D, P, d_left, d_right, steps=3):
     ctx.close()
     upd = W * H * D * P * 2
     return {"workload": "plain pair 1600x1067 D=256 with 32-bit aggregates (uint16 cost volume, "
-                        "int32 aggregate volume, generic recurrence)",
+                        "32-bit path costs and sums, excess planes in the int32 volume's room)",
             "ms_per_pair": round(t * 1e3, 3), "gupdates_per_s": round(upd / t / 1e9, 3),
             "kernel_ms": prof, "device_bytes": plan["pair_bytes"],
             "aggregate_bytes": plan["aggregate_bytes"]}
@@ -682,7 +683,7 @@ def write_traffic(fetch_dir, write_dir, copy_bytes=2 << 30, paths=8):
     sweep = lambda k, phase: "path_kernel<4, unsigned short, %d, " % phase in k
     planes = any("excess_kernel<16, 16, " in k for k, _ in fetch)
     if planes:
-        kinds = (("cost", lambda k: sweep(k, 3), cells, 1),
+        kinds = (("cost", lambda k: "band_cost_kernel<16, 16, " in k, cells, 1),
                  ("excess", lambda k: "excess_kernel<16, 16, " in k,
                   int(3.25 * (paths // 2) * cells), 1),
                  ("winner", lambda k: "winner_kernel<16, 16, " in k, (1 + paths // 2) * cells, 1))
@@ -899,7 +900,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBPS,
                      "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBPS, 4),
                      "traffic": traffic,
-                     "kernel": "path sweeps of one pair (sgm::path_kernel cost pass, "
+                     "kernel": "path sweeps of one pair (sgm::band_cost_kernel, "
                                "sgm::excess_kernel, sgm::winner_kernel)",
                      "sweeps": ["auto", "sequential", "paired", "planes"][schedule],
                      "launches_per_step": path_launches,

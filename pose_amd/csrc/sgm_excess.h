@@ -21,7 +21,8 @@
 // 256 disparities; 45 and 8 at 64.
 //
 // Measured against one launch per seven directions and a fused last sweep with
-// one line per wave (both matching directions, census 9x7): 640x480 D=64
+// one line per wave (both matching directions, census 9x7; cost and census kernels
+// of that time on both sides): 640x480 D=64
 // 653 -> 304 us a pair, 1600x1067 D=256 4.03 -> 3.11 ms with pair sweeps (4.24
 // with one plane per path: at that size HBM traffic decides, 26 or 19 bytes per
 // cell), 2901x2175 D=350 24.7 -> 18.6 ms; FP32 ZNCC 1600x1067 D=192 against
