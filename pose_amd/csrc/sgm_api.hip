@@ -2126,6 +2126,8 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     A.seg = band_segment(p, (int64_t)nd * w * h);
     A.split = (h * band_segments(w, A.seg) + 64 / lanes - 1) / (64 / lanes);
     A.total = nd * A.split;
+    A.stream = B.nplanes && (int64_t)nd * w * h * Dp * ((cost_u8(p) ? 1 : 2) + B.nplanes) >
+                                kStreamBytes;
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
     if ((rc = launch_band(ctx, Dp, p, pj, A))) return rc;
   }

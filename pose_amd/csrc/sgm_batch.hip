@@ -286,6 +286,7 @@ static int phased_enqueue(sgm_batch *b) {
       A.seg = g.seg;
       A.total = g.total_lines[3];
       A.wave_begin = g.line_begin[3];
+      A.stream = g.nt;
       if ((rc = launch_band(ctx, g.Dp, p, pj, A, st))) return rc;
       ExcessArgs E = excess_args(p, g.njobs, b->nplanes);
       for (int k = 0; k < E.ndirs; k++) {

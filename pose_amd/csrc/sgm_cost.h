@@ -15,7 +15,9 @@
 // AD-census 11x11 1201x801 D=97 754 -> 175 us, census 5x5 1200x900 D=700 2806 ->
 // 479 us, uint16 census 9x7 1024x768 D=128 385 -> 85 us; against a sliding
 // window with one segment per wave: census 9x7 640x480 D=64 45 -> 20 us,
-// 1600x1067 D=256 302 -> 246 us, 2901x2175 D=350 1866 -> 1387 us (3.5 TB/s).
+// 1600x1067 D=256 302 -> 246 us, 2901x2175 D=350 1866 -> 1387 us (3.5 TB/s), with
+// stores past the caches (where the sweeps' volumes exceed 1 GiB) 202 and 969 us;
+// below that size the sweeps want the costs in them (640x480: 252 -> 284 us a pair).
 #pragma once
 
 namespace sgm {
@@ -26,6 +28,7 @@ struct BandArgs {
   const int *wave_begin; // jobs in a device table: first wave of each job
   int seg;               // pixels per row segment
   int gradient;          // difference of the gray gradients instead of the grays
+  int stream;            // volumes far beyond the caches: the stores pass them by
   // AD-census, census-gradient: value = (wa * ham + wb * min(difference, cap) + half) / den as
   // a multiplication by `magic` and a shift (band_division)
   uint32_t wa, wb, half, cap, magic;
@@ -167,8 +170,10 @@ struct BandCost {
         }
       }
     }
-    bstore_dwords<OUT16 ? 2 * ND : ND, POL_DEFAULT>(out, make_rsrc(row, kExcessRange),
-                                                    s < len ? off : kExcessDrop);
+    const __amdgpu_buffer_rsrc_t to = make_rsrc(row, kExcessRange);
+    const int at = s < len ? off : kExcessDrop;
+    if (A.stream) bstore_dwords<OUT16 ? 2 * ND : ND, POL_NT>(out, to, at);
+    else bstore_dwords<OUT16 ? 2 * ND : ND, POL_DEFAULT>(out, to, at);
     // the targets move by one column
     Target e;
     const Target &end = win[REV ? 0 : R - 1];
