@@ -932,8 +932,6 @@ ExcessArgs excess_args(const sgm_params *p, int njobs, int planes) {
   return E;
 }
 
-int lines_of(int cls, int w, int h) { return cls == 0 ? h : cls == 1 ? w : w + h - 1; }
-
 int launch_path(sgm_context *ctx, int R, int sum_bytes, int mode, const PathJobs &jobs,
                 const PathArgs &A, int phase, int waves, hipStream_t stream) {
   ProfileScope ps(ctx, phase == PHASE_FIRST ? "path_first"
@@ -1689,79 +1687,36 @@ int launch_esgm_verify(sgm_context *ctx, int R, const SummaryJobs &J, int slots)
   return launch_check("compact verification kernel");
 }
 
-// Compact plan for `nd` matching directions (GpuCandidateStereo.execute/run,
-// GpuCandidateStereo.java:49-171, 190-335): proposal sweeps and sum sweeps
-// over every path and strip, certification, exact verification of the rest in
-// groups that fit the budget, then selection of every pixel from its summary.
-// Same contract as run_directions.
-}  // namespace
-
-namespace sgm {
-
-int line_length(int dx, int dy, int line, int w, int h) {
-  if (dy == 0) return w;
-  if (dx == 0) return h;
-  // the diagonal line enumeration of line_start
-  const int x = line < w ? line : (dx > 0 ? 0 : w - 1);
-  const int y = line < w ? (dy > 0 ? 0 : h - 1) : (dy > 0 ? line - w + 1 : h - 2 - (line - w));
-  return std::min(dx > 0 ? w - x : x + 1, dy > 0 ? h - y : y + 1);
-}
-
-int wave_length(int dx, int dy, int wave, int per, int w, int h) {
-  const int lines = lines_of(dy == 0 ? 0 : dx == 0 ? 1 : 2, w, h);
-  int n = 0;
-  for (int l = wave * per; l < std::min(lines, (wave + 1) * per); l++)
-    n = std::max(n, line_length(dx, dy, l, w, h));
-  return n;
-}
-
-void longest_first(const std::vector<int> &len, int maxlen, std::vector<int> &order) {
-  // counting sort by length, descending; lines of equal length in line order
-  std::vector<int> start((size_t)maxlen + 2, 0);
-  for (int n : len) start[maxlen - n + 1]++;  // bucket maxlen - n: longest first
-  for (int i = 1; i <= maxlen + 1; i++) start[i] += start[i - 1];
-  order.assign(len.size(), 0);
-  for (size_t g = 0; g < len.size(); g++) order[start[maxlen - len[g]]++] = (int)g;
-}
-
-}  // namespace sgm
-
-namespace {
-
-// Longest-first dispatch order of the waves of a launch over a w x h pair (nd
-// matching directions; waves [begin[k], begin[k] + nd * split[k]) sweep
-// direction (dx[k], dy[k]), `per` neighbouring lines each, matching direction
-// m's from begin[k] + m * split[k]), in a device buffer cached by shape.  A
+// Longest-first dispatch order of a launch's waves in a device buffer of its own
+// (`name`, one per kind of launch), cached with the layout it holds for.  A
 // launch with several times more lines than resident waves otherwise ends on
 // long lines dispatched last (seven directions with one line per wave at
 // 1600x1067 D=256: 2.48 -> 2.30 ms).  Null, for the natural order, when the
 // buffer does not fit the budget.
-static const int *line_order(sgm_context *ctx, const char *name, int ndirs, const int *dx,
-                             const int *dy, const int *split, const int *begin, int total, int w,
-                             int h, int nd, int per = 1) {
+static const int *line_order(sgm_context *ctx, const std::string &name, const WaveLayout &layout) {
   sgm_context::LineOrder &lo = ctx->line_orders[name];
-  const int key[7] = {w, h, nd, ndirs, dx[0], dy[0], per};
   Buffer &buf = ctx->buffers[name];
-  if (buf.ptr && memcmp(lo.key, key, sizeof key) == 0) return (const int *)buf.ptr;
-  const size_t bytes = (size_t)total * sizeof(int);
+  if (buf.ptr && lo.layout == layout) return (const int *)buf.ptr;
+  lo.layout = WaveLayout{};
+  const size_t bytes = (size_t)layout.total * sizeof(int);
   if (bytes > buf.cap && ctx->allocated - (int64_t)buf.cap + (int64_t)bytes > ctx->budget)
     return nullptr;
   if (buf.ensure(ctx, bytes, "line order")) return nullptr;
-  std::vector<int> len((size_t)total);
-  for (int k = 0; k < ndirs; k++)
-    for (int m = 0; m < nd; m++)
-      for (int l = 0; l < split[k]; l++)
-        len[(size_t)begin[k] + (size_t)m * split[k] + l] = wave_length(dx[k], dy[k], l, per, w, h);
-  longest_first(len, std::max(w, h), lo.host);
+  wave_order(layout, lo.host);
   hipError_t e = hipMemcpyAsync(buf.ptr, lo.host.data(), bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  memcpy(lo.key, key, sizeof key);
+  lo.layout = layout;
   return (const int *)buf.ptr;
 }
 
+// Compact plan for `nd` matching directions (GpuCandidateStereo.execute/run,
+// GpuCandidateStereo.java:49-171, 190-335): proposal sweeps and sum sweeps
+// over every path and strip, certification, exact verification of the rest in
+// groups that fit the budget, then selection of every pixel from its summary.
+// Same contract as run_directions.
 int run_directions_esgm(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuffers &B,
                         const int *slots, int nd, int out_slot, uint8_t *reasons,
                         uint8_t *boundary) {
@@ -2142,15 +2097,12 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     ExcessArgs E = excess_args(p, nd, B.nplanes);
     int lanes = 0, er = 0;
     excess_shape(Dp, lanes, er);
-    const int per = 64 / lanes;
-    for (int k = 0; k < E.ndirs; k++) {
-      const int cls = E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2;
-      E.split[k] = (lines_of(cls, w, h) + per - 1) / per;
-      E.begin[k] = E.total;
-      E.total += nd * E.split[k];
-    }
-    E.order = line_order(ctx, "excess_order", E.ndirs, E.dx, E.dy, E.split, E.begin, E.total, w, h,
-                         nd, per);
+    const WaveLayout layout = wave_layout(E.ndirs, E.dx, E.dy, w, h, nd, 64 / lanes);
+    memcpy(E.split, layout.split, sizeof E.split);
+    memcpy(E.begin, layout.begin, sizeof E.begin);
+    E.total = layout.total;
+    E.order = line_order(ctx, "excess_order" + std::to_string(p->directions) +
+                                  (E.pairs ? "_pairs" : ""), layout);
     if (interrupted()) return fail(SGM_ERR_INTERRUPTED, "GPU SGM interrupted");
     const bool wide = aggregate_bytes(p) == 4;
     if ((rc = wide ? launch_excess32(ctx, Dp, stream, pj, E)
@@ -2179,10 +2131,8 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
       // (its first direction when dir == 1)
       static const char *pair_names[8] = {"", "pair_order1", "", "pair_order3", "", "pair_order5"};
       PathArgs Aa = dir_args(dir), Ab = dir_args(dir + 1);
-      const int dxs[2] = {Aa.dx, Ab.dx}, dys[2] = {Aa.dy, Ab.dy}, splits[2] = {Aa.split, Ab.split};
-      const int begins[2] = {0, Aa.total_lines};
-      Aa.order = line_order(ctx, pair_names[dir], 2, dxs, dys, splits, begins,
-                            Aa.total_lines + Ab.total_lines, w, h, nd);
+      const int dxs[2] = {Aa.dx, Ab.dx}, dys[2] = {Aa.dy, Ab.dy};
+      Aa.order = line_order(ctx, pair_names[dir], wave_layout(2, dxs, dys, w, h, nd, 1));
       if ((rc = launch_path_pair(ctx, R, mode, dir == 1 ? PHASE_FIRST : PHASE_MID, pj, Aa, pjb, Ab,
                                  waves)))
         return rc;
@@ -2200,9 +2150,7 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     if (Ad.cls == 2) {  // diagonal lines differ in length: longest first
       static const char *dir_names[8] = {"", "", "", "", "dir_order4", "dir_order5", "dir_order6",
                                          "dir_order7"};
-      const int zero = 0;
-      Ad.order = line_order(ctx, dir_names[dir], 1, &Ad.dx, &Ad.dy, &Ad.split, &zero,
-                            Ad.total_lines, w, h, nd);
+      Ad.order = line_order(ctx, dir_names[dir], wave_layout(1, &Ad.dx, &Ad.dy, w, h, nd, 1));
     }
     if ((rc = launch_path(ctx, R, sb, m, jobs, Ad, phase, waves))) return rc;
     dir++;

@@ -12,6 +12,7 @@
 
 #include "../../include/sgm_hip.h"
 #include "sgm_kernels.h"
+#include "sgm_order.h"
 
 struct sgm_context;
 
@@ -75,13 +76,6 @@ bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h,
 int64_t schedule_bytes(const sgm_params *p, int w, int h, int schedule);
 int sweep_schedule(const sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                    int64_t budget);
-int lines_of(int cls, int w, int h);
-// length of line `line` of direction (dx, dy) in a w x h image (line_start)
-int line_length(int dx, int dy, int line, int w, int h);
-// longest of the `per` lines of wave `wave`
-int wave_length(int dx, int dy, int wave, int per, int w, int h);
-// the indices of `len` by length, longest first, equal lengths in index order
-void longest_first(const std::vector<int> &len, int maxlen, std::vector<int> &order);
 struct HostCopy {
   void *dst;
   const void *src;
@@ -203,11 +197,10 @@ struct sgm_context {
   bool last_compact = false;
   int sweeps = SGM_SWEEPS_AUTO;  // sgm_set_sweeps
   // longest-first orders of a launch's waves, by buffer name: the host copy and
-  // the (w, h, matching directions, directions, first dx, dy, lines per wave)
-  // it is for
+  // the waves it is for
   struct LineOrder {
     std::vector<int> host;
-    int key[7] = {0, 0, 0, 0, 0, 0, 0};
+    sgm::WaveLayout layout = {};
   };
   std::map<std::string, LineOrder> line_orders;
   int last_sweeps = SGM_SWEEPS_SEQUENTIAL;
