@@ -607,6 +607,11 @@ struct PairSweep : ExcessLines<LANES, R, CB, NT> {
     for (; s0 >= 0; s0 -= SEG) {
       mf = this->penalty(g, gp);
       mb = this->penalty(g, gn);
+      // (lanes past the padded row keep no bytes: a pad's, not the minimum's)
+      if constexpr (LANES > 16) {
+#pragma unroll
+        for (int i = 0; i < ND; i++) kept[i] |= this->beyond;
+      }
       fwd.restore(kept);
       // the next segment's state and pixels, one segment ahead
       st = this->prow + (ptrdiff_t)(s0 - SEG) * this->pstep;
