@@ -11,7 +11,8 @@
 //
 // The proposal pass runs every direction in one launch (a direction writes only
 // its own proposals); the verification pass too, adding with 32-bit atomics on
-// packed pairs (no half passes 65535, so none carries).  Both are bound by VALU,
+// packed pairs: a cell's sum stays within 16 bits (paths * (512 + P2)), a pad
+// cell's would not and is left out, so no half carries.  Both are bound by VALU,
 // 120 instructions a wave and step, 190 with two proposals, issued at about 85%
 // of the rate.  The sum pass accumulates, so direction by direction, and its one
 // or two waves per SIMD are bound by their own issue; four pixels' proposals are
@@ -348,7 +349,7 @@ struct CompactLine {
       uint32_t *row = reinterpret_cast<uint32_t *>(J.verify + (size_t)(sl - J.lo) * J.Dp) + own;
 #pragma unroll
       for (int i = 0; i < NP; i++)
-        __hip_atomic_fetch_add(row + i * lanes, L[i], __ATOMIC_RELAXED,
+        __hip_atomic_fetch_add(row + i * lanes, L[i] & keep[i], __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
     }
   }
