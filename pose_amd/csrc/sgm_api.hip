@@ -2598,9 +2598,13 @@ namespace {
 
 // Writes the disparities straight into the caller's maps where those are
 // float-aligned and share no byte with another buffer of the call (the maps are
-// written before the other outputs); elsewhere they are copied at the end.
+// written before the other outputs); elsewhere they are copied at the end.  The
+// resident and compact plans select every pixel of both maps in their last
+// launch, past the last interruption check; the streamed plan does so strip by
+// strip and can stop in between, so it copies.
 void direct_disparities(PairBuffers &B, size_t n, const void *const *others, const size_t *bytes,
                         int count, void *d_dl, void *d_dr) {
+  if (B.strip_rows) return;
   void *out[2] = {d_dl, d_dr};
   for (int d = 0; d < 2; d++) {
     const uintptr_t a = (uintptr_t)out[d];
