@@ -18,6 +18,8 @@
 // 1600x1067 D=256 302 -> 246 us, 2901x2175 D=350 1866 -> 1387 us (3.5 TB/s), with
 // stores past the caches (where the sweeps' volumes exceed 1 GiB) 202 and 969 us;
 // below that size the sweeps want the costs in them (640x480: 252 -> 284 us a pair).
+// The 20 bytes of a lane at 16 x 20 and 32 x 20 take two stores that each cover parts
+// of a 64-byte granule, so there the caches join them: 2000x1400 D=320 0.72 -> 0.60 ms.
 #pragma once
 
 namespace sgm {
@@ -172,7 +174,7 @@ struct BandCost {
     }
     const __amdgpu_buffer_rsrc_t to = make_rsrc(row, kExcessRange);
     const int at = s < len ? off : kExcessDrop;
-    if (A.stream) bstore_dwords<OUT16 ? 2 * ND : ND, POL_NT>(out, to, at);
+    if (R != 20 && A.stream) bstore_dwords<OUT16 ? 2 * ND : ND, POL_NT>(out, to, at);
     else bstore_dwords<OUT16 ? 2 * ND : ND, POL_DEFAULT>(out, to, at);
     // the targets move by one column
     Target e;

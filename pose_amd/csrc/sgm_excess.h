@@ -47,8 +47,9 @@ namespace sgm {
 constexpr int kMaxExcessDirs = 8;
 constexpr uint32_t kExcessInf = 0x70007000u;
 // buffer range of the excess sweeps' accesses and the offset of a dropped one
+// (further planes and row tails lie behind it, below 2^31)
 constexpr uint32_t kExcessRange = 0x7F000000u;
-constexpr int kExcessDrop = 0x7FFFFF00;
+constexpr int kExcessDrop = 0x7F000000;
 
 // Lanes per line and disparities per lane for a padded row of Dp cells (Dp a
 // multiple of 64, at most 1024); false: no shape.  R divides Dp, so a lane lies
@@ -139,6 +140,32 @@ __device__ __forceinline__ void bstore_dwords(const uint32_t *src, __amdgpu_buff
     if constexpr (N > 4) bstore_dwords<N - 4, POL>(src + 4, r, off + 16);
   }
 }
+
+// A lane's R bytes of a plane row of LANES * R: at l * R, but 20 bytes take two
+// accesses, which side by side would each cover parts of every 64-byte granule, so
+// there the row holds the first 16 bytes of all lanes and then their last 4.
+// 2000x1400 D=320, 20 bytes side by side against this: a plane per path 10.6 -> 6.1
+// ms and its winner search 3.2 -> 2.5, a plane per pair 5.9 -> 5.2 and 1.8 -> 1.5.
+template <int LANES, int R>
+struct PlaneRow {
+  static constexpr bool SPLIT = R == 20;
+  static constexpr int ND = R / 4, HEAD = SPLIT ? 4 : ND;
+  static __device__ __forceinline__ int head(int l) { return l * HEAD * 4; }
+  // bytes from the head to the tail
+  static __device__ __forceinline__ int tail(int l) { return (LANES - l) * 16 + l * 4; }
+  template <int POL>
+  static __device__ __forceinline__ void load(uint32_t *dst, __amdgpu_buffer_rsrc_t r, int off,
+                                              int l) {
+    bload_dwords<HEAD, POL>(dst, r, off);
+    if constexpr (SPLIT) bload_dwords<1, POL>(dst + 4, r, off + tail(l));
+  }
+  template <int POL>
+  static __device__ __forceinline__ void store(const uint32_t *src, __amdgpu_buffer_rsrc_t r,
+                                               int off, int l) {
+    bstore_dwords<HEAD, POL>(src, r, off);
+    if constexpr (SPLIT) bstore_dwords<1, POL>(src + 4, r, off + tail(l));
+  }
+};
 
 // Minimum of three packed pairs; every half non-negative and below 0x7C00.
 __device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
@@ -406,7 +433,7 @@ struct ExcessLines {
     const int rel = len > 0 ? p0 - base : 0;
     const bool inside = l * R < J.Dp;
     coff = inside ? (rel * J.Dp + l * R) * CB : kExcessDrop;
-    poff = inside ? rel * A.planes * J.Dp + l * R : kExcessDrop;
+    poff = inside ? rel * A.planes * J.Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
     cstep = (ptrdiff_t)step * J.Dp * CB;
     pstep = (ptrdiff_t)step * J.Dp * A.planes;
     crow = J.cost + (ptrdiff_t)base * J.Dp * CB;
@@ -422,7 +449,8 @@ struct ExcessLines {
     bload_dwords<ND * CB, POL_DEFAULT>(dst, make_rsrc(row, kExcessRange), in ? coff : kExcessDrop);
   }
   __device__ __forceinline__ void store(const uint32_t *src, uint8_t *row, bool in) const {
-    bstore_dwords<ND, POL>(src, make_rsrc(row, kExcessRange), in ? poff : kExcessDrop);
+    PlaneRow<LANES, R>::template store<POL>(src, make_rsrc(row, kExcessRange),
+                                            in ? poff : kExcessDrop, lane_id() % LANES);
   }
   // gray | mask << 8 of the pixel of step s (0, an unusable pixel, off the line)
   __device__ __forceinline__ int pixel(int s) const {
@@ -532,6 +560,12 @@ struct PairSweep : ExcessLines<LANES, R, CB, NT> {
     this->store(out, st, in);
   }
 
+  __device__ __forceinline__ void keep_load(uint32_t *kept, bool in) const {
+    PlaneRow<LANES, R>::template load<POL_DEFAULT>(kept, make_rsrc(st, kExcessRange),
+                                                   in ? this->poff : kExcessDrop,
+                                                   lane_id() % LANES);
+  }
+
   template <int JJ>
   __device__ __forceinline__ void ahead(int s) {
     uint32_t c[R / 2], e[R / 2];
@@ -602,8 +636,7 @@ struct PairSweep : ExcessLines<LANES, R, CB, NT> {
     ld = this->crow + (ptrdiff_t)(s0 - 1) * this->cstep;
     uint32_t kept[ND];
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the kept states are in memory
-    bload_dwords<ND, POL_DEFAULT>(kept, make_rsrc(st, kExcessRange),
-                                  s0 < this->len ? this->poff : kExcessDrop);
+    keep_load(kept, s0 < this->len);
     for (; s0 >= 0; s0 -= SEG) {
       mf = this->penalty(g, gp);
       mb = this->penalty(g, gn);
@@ -615,8 +648,7 @@ struct PairSweep : ExcessLines<LANES, R, CB, NT> {
       fwd.restore(kept);
       // the next segment's state and pixels, one segment ahead
       st = this->prow + (ptrdiff_t)(s0 - SEG) * this->pstep;
-      bload_dwords<ND, POL_DEFAULT>(kept, make_rsrc(st, kExcessRange),
-                                    s0 >= SEG && s0 - SEG < this->len ? this->poff : kExcessDrop);
+      keep_load(kept, s0 >= SEG && s0 - SEG < this->len);
       const int s = s0 - SEG + i;
       g = this->pixel(s);
       gp = this->pixel(s - 1);
@@ -689,7 +721,8 @@ struct WinnerSearch {
     bload_dwords<ND * CB, POL>(r.c, make_rsrc(cost, kExcessRange), coff);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(planes, kExcessRange);
 #pragma unroll
-    for (int k = 0; k < NPL; k++) bload_dwords<ND, POL>(r.pl[k], rs, poff + k * Dp);
+    for (int k = 0; k < NPL; k++)
+      PlaneRow<LANES, R>::template load<POL>(r.pl[k], rs, poff + k * Dp, lane_id() % LANES);
   }
 
   // Aggregates of one lane's cells, invalid and pad cells 0xFFFF.
@@ -764,7 +797,7 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner_kernel(PathJobs jobs
   const uint8_t *cost = V.cost + ((size_t)y * V.w + x0) * Dp * CB;
   const uint8_t *planes = V.planes + ((size_t)y * V.w + x0) * Dp * NPL;
   const int coff = inside ? (g * Dp + l * R) * CB : kExcessDrop;
-  const int poff = inside ? g * NPL * Dp + l * R : 0x7F000000;
+  const int poff = inside ? g * NPL * Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
   uint32_t kpk[NP];
 #pragma unroll
   for (int i = 0; i < NP; i++) {
@@ -774,14 +807,14 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner_kernel(PathJobs jobs
   uint8_t *row = cells[wv];
   const int own = lane * R * 2, line = g * LANES * R * 2;
   typename WS::Row cur;
-  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : 0x7F000000, Dp);
+  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, Dp);
   for (int i = 0; i < count; i += NL) {
     uint32_t S[NP];
     WS::sums(cur, beyond, paths, S);
     cost += NL * Dp * CB;
     planes += NL * Dp * NPL;
     const bool next = i + NL + g < count;
-    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : 0x7F000000, Dp);
+    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, Dp);
 #pragma unroll
     for (int j = 0; j < NP; j += 2)
       *reinterpret_cast<uint2 *>(row + own + 4 * j) = make_uint2(S[j], S[j + 1]);
@@ -855,11 +888,11 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner32_kernel(PathJobs jo
   const uint8_t *cost = V.cost + ((size_t)y * V.w + x0) * Dp * 2;
   const uint8_t *planes = V.planes + ((size_t)y * V.w + x0) * Dp * 4;
   const int coff = inside ? (g * Dp + l * R) * 2 : kExcessDrop;
-  const int poff = inside ? g * 4 * Dp + l * R : 0x7F000000;
+  const int poff = inside ? g * 4 * Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
   uint32_t *own = cells[wv] + lane * R;
   const uint32_t *line = cells[wv] + g * LANES * R;
   typename WS::Row cur;
-  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : 0x7F000000, Dp);
+  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, Dp);
   for (int i = 0; i < count; i += NL) {
     uint32_t S[R];  // invalid and pad cells: none
     uint32_t value = none;
@@ -876,7 +909,7 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner32_kernel(PathJobs jo
     cost += NL * Dp * 2;
     planes += NL * Dp * 4;
     const bool next = i + NL + g < count;
-    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : 0x7F000000, Dp);
+    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, Dp);
 #pragma unroll
     for (int j = 0; j < R; j += 4)
       *reinterpret_cast<uint4 *>(own + j) = make_uint4(S[j], S[j + 1], S[j + 2], S[j + 3]);

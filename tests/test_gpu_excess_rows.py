@@ -65,3 +65,30 @@ def test_full_rows_equal_the_aggregate(case):
     for k in ("reasons", "boundary"):
         assert np.array_equal(a[k], b[k]), k
     assert a["stats"] == b["stats"]
+
+
+def test_rows_of_20_bytes_a_lane_cost_what_other_rows_do():
+    """One plane per path beyond the caches: a cell of the 320-disparity shape (20
+    bytes a lane, two accesses) takes no longer than 1.3 of a 384-disparity one."""
+    per_cell = {}
+    for D in (320, 384):
+        w, h = 1600, 900
+        p = sgm.SgmParams(window_w=9, window_h=7, disparities=D, min_disparity=0, cost=0, p1=10,
+                          p2=150, edge_scale=32, directions=8, aggregate_bytes=0,
+                          census_weight=500, ad_truncation=30, gradient_truncation=60, reserved=0,
+                          uniqueness=0.03, lr_threshold=1.0)
+        left, right, _ = synth.stereo_pair(w, h, D, 0, seed=D)
+        ctx = sgm.Context(0)
+        try:
+            ctx.match_pair(p, left, right)
+            ctx.set_profiling(True)
+            runs = []
+            for _ in range(5):
+                ctx.profile()
+                ctx.match_pair(p, left, right)
+                runs.append(ctx.profile()["device_kernel_milliseconds"]["path_excess"]["total_ms"])
+            per_cell[D] = min(runs) / D
+        finally:
+            ctx.close()
+    print("excess sweeps, us per disparity:", per_cell, flush=True)
+    assert per_cell[320] <= 1.3 * per_cell[384], per_cell
