@@ -1043,14 +1043,20 @@ struct PairBuffers {
 
 }  // namespace
 
+// Bytes that `budget` leaves for a resident pair's planes.
+static int64_t plane_room(const sgm_params *p, int w, int h, int64_t budget) {
+  const int64_t cells = 2 * (int64_t)w * h * padded_disparities(p->disparities);
+  return budget - (pair_bytes(p, w, h, true) - cells * aggregate_bytes(p));
+}
+
 // Device bytes a sweep schedule adds to pair_bytes(p, w, h, true): the second
 // partial aggregate volumes of paired sweeps, or the excess planes of both
 // matching directions (one byte per cell and plane) in place of the aggregates.
-int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule) {
+int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule, int64_t budget) {
   const int64_t cells = 2 * (int64_t)w * h * padded_disparities(p->disparities);
   if (schedule == SGM_SWEEPS_PAIRED) return cells * aggregate_bytes(p);
   if (schedule == SGM_SWEEPS_PLANES)
-    return cells * (excess_plane_count(p, cells) - aggregate_bytes(p));
+    return cells * (excess_plane_count(p, cells, plane_room(p, w, h, budget)) - aggregate_bytes(p));
   return 0;
 }
 
@@ -1082,10 +1088,13 @@ bool sgm::schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, i
 // Planes per pixel of 8 paths over `cells` cells of all matching directions: one
 // per path, or one per pair of opposite paths (PairSweep, sgm_excess.h) where
 // their summed excesses fit a byte and the volumes are so far beyond the caches
-// that HBM traffic counts.
-int sgm::excess_plane_count(const sgm_params *p, int64_t cells) {
-  const bool pairs = 2 * effective_p2(p) <= 255 && cells * (1 + kMaxExcessDirs) > kPairBytes;
-  return pairs ? kMaxExcessDirs / 2 : kMaxExcessDirs;
+// that HBM traffic counts, or `room` bytes hold no more than the seven path-cost
+// planes that a budget may be sized for (640x480 D=64 in pairs 0.29 ms, with the
+// paired aggregates that would be next 0.73).
+int sgm::excess_plane_count(const sgm_params *p, int64_t cells, int64_t room) {
+  const bool far = cells * (1 + kMaxExcessDirs) > kPairBytes;
+  const bool tight = room >= cells * (kMaxExcessDirs - 1) && room < cells * kMaxExcessDirs;
+  return 2 * effective_p2(p) <= 255 && (far || tight) ? kMaxExcessDirs / 2 : kMaxExcessDirs;
 }
 
 // Excess planes per pixel of a pair on the resident plan under `schedule` (0:
@@ -1096,9 +1105,10 @@ int sgm::excess_plane_count(const sgm_params *p, int64_t cells) {
 // winner32_kernel), but no aggregate goes through memory, and 19 + 8 bytes a
 // cell replace 74 of eight sequential sweeps.
 int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
-                       bool cost_volume) {
+                       bool cost_volume, int64_t budget) {
   if (schedule == SGM_SWEEPS_PLANES)
-    return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities));
+    return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities),
+                              plane_room(p, w, h, budget));
   if (ctx->keep_volumes || !cost_volume || !excess_possible(p, w, h)) return 0;
   if (schedule == SGM_SWEEPS_PAIRED) return p->directions == 4 ? 4 : 0;
   return aggregate_bytes(p) == 4 && ctx->sweeps != SGM_SWEEPS_SEQUENTIAL &&
@@ -1118,7 +1128,7 @@ int sgm::sweep_schedule(const sgm_context *ctx, const sgm_params *p, int w, int 
   for (int sched : {SGM_SWEEPS_PLANES, SGM_SWEEPS_PAIRED}) {
     if (sched == SGM_SWEEPS_PLANES && want == SGM_SWEEPS_PAIRED) continue;
     if (schedule_applies(ctx, p, w, h, sched, cost_volume) &&
-        base + schedule_bytes(p, w, h, sched) <= budget)
+        base + schedule_bytes(p, w, h, sched, budget) <= budget)
       return sched;
   }
   return SGM_SWEEPS_SEQUENTIAL;
@@ -1172,11 +1182,12 @@ static std::vector<std::pair<std::string, size_t>> pair_buffer_list(const sgm_pa
 // Device bytes the context holds once ensure_pair_buffers has served the pair
 // on the resident plan with sweep schedule `schedule`: each of the pair's
 // buffers grows to its size when its cached capacity is smaller, every other
-// cached buffer stays as it is (`fresh`: no cached buffers).
+// cached buffer stays as it is (`fresh`: no cached buffers).  Planes are counted
+// as an ample budget has them.
 int64_t sgm::resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h,
                                 bool cost_volume, int schedule, bool fresh) {
   int64_t total = fresh ? 0 : ctx->allocated;
-  const int planes = excess_planes(ctx, p, w, h, schedule, cost_volume);
+  const int planes = excess_planes(ctx, p, w, h, schedule, cost_volume, INT64_MAX);
   for (const auto &b : pair_buffer_list(p, w, h, true, cost_volume, schedule, planes)) {
     if (fresh) {
       total += (int64_t)b.second;
@@ -1201,7 +1212,7 @@ int ensure_pair_buffers(sgm_context *ctx, const sgm_params *p, int w, int h, Pai
   const bool recompute = !rows && recompute_cost(ctx, p, w, h);
   const int schedule =
       rows ? SGM_SWEEPS_SEQUENTIAL : sweep_schedule(ctx, p, w, h, !recompute, ctx->budget);
-  const int planes = rows ? 0 : excess_planes(ctx, p, w, h, schedule, !recompute);
+  const int planes = rows ? 0 : excess_planes(ctx, p, w, h, schedule, !recompute, ctx->budget);
   int rc;
 #define ENSURE(name, bytes)                                                   \
   if ((rc = ctx->buffers[name].ensure(ctx, (bytes), name)) != SGM_OK) return rc;

@@ -68,12 +68,12 @@ int64_t pair_bytes(const sgm_params *p, int w, int h, bool cost_volume);
 int64_t resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                            int schedule, bool fresh);
 bool excess_possible(const sgm_params *p, int w, int h);
-int excess_plane_count(const sgm_params *p, int64_t cells);
+int excess_plane_count(const sgm_params *p, int64_t cells, int64_t room = INT64_MAX);
 int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
-                  bool cost_volume);
+                  bool cost_volume, int64_t budget);
 bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                       bool cost_volume);
-int64_t schedule_bytes(const sgm_params *p, int w, int h, int schedule);
+int64_t schedule_bytes(const sgm_params *p, int w, int h, int schedule, int64_t budget);
 int sweep_schedule(const sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                    int64_t budget);
 struct HostCopy {
