@@ -152,18 +152,18 @@ struct PlaneRow {
   static constexpr int ND = R / 4, HEAD = SPLIT ? 4 : ND;
   static __device__ __forceinline__ int head(int l) { return l * HEAD * 4; }
   // bytes from the head to the tail
-  static __device__ __forceinline__ int tail(int l) { return (LANES - l) * 16 + l * 4; }
+  static __device__ __forceinline__ int tail(int l) { return SPLIT ? (LANES - l) * 16 + l * 4 : 0; }
   template <int POL>
   static __device__ __forceinline__ void load(uint32_t *dst, __amdgpu_buffer_rsrc_t r, int off,
-                                              int l) {
+                                              int tail) {
     bload_dwords<HEAD, POL>(dst, r, off);
-    if constexpr (SPLIT) bload_dwords<1, POL>(dst + 4, r, off + tail(l));
+    if constexpr (SPLIT) bload_dwords<1, POL>(dst + 4, r, off + tail);
   }
   template <int POL>
   static __device__ __forceinline__ void store(const uint32_t *src, __amdgpu_buffer_rsrc_t r,
-                                               int off, int l) {
+                                               int off, int tail) {
     bstore_dwords<HEAD, POL>(src, r, off);
-    if constexpr (SPLIT) bstore_dwords<1, POL>(src + 4, r, off + tail(l));
+    if constexpr (SPLIT) bstore_dwords<1, POL>(src + 4, r, off + tail);
   }
 };
 
@@ -402,7 +402,7 @@ struct ExcessLines {
   const uint32_t *tab;
   int len, maxlen, minlen;      // this lane's line, longest and shortest of the wave
   int p0, step;                 // first pixel of this lane's line, pixels per step
-  int coff, poff;               // this lane's offsets in the wave's cost / plane rows
+  int coff, poff, ptail;        // this lane's offsets in the wave's cost / plane rows
   const uint8_t *crow;          // the wave's cost and plane rows of step 0
   uint8_t *prow;
   ptrdiff_t cstep, pstep;
@@ -434,6 +434,7 @@ struct ExcessLines {
     const bool inside = l * R < J.Dp;
     coff = inside ? (rel * J.Dp + l * R) * CB : kExcessDrop;
     poff = inside ? rel * A.planes * J.Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
+    ptail = PlaneRow<LANES, R>::tail(l);
     cstep = (ptrdiff_t)step * J.Dp * CB;
     pstep = (ptrdiff_t)step * J.Dp * A.planes;
     crow = J.cost + (ptrdiff_t)base * J.Dp * CB;
@@ -450,7 +451,7 @@ struct ExcessLines {
   }
   __device__ __forceinline__ void store(const uint32_t *src, uint8_t *row, bool in) const {
     PlaneRow<LANES, R>::template store<POL>(src, make_rsrc(row, kExcessRange),
-                                            in ? poff : kExcessDrop, lane_id() % LANES);
+                                            in ? poff : kExcessDrop, ptail);
   }
   // gray | mask << 8 of the pixel of step s (0, an unusable pixel, off the line)
   __device__ __forceinline__ int pixel(int s) const {
@@ -562,8 +563,7 @@ struct PairSweep : ExcessLines<LANES, R, CB, NT> {
 
   __device__ __forceinline__ void keep_load(uint32_t *kept, bool in) const {
     PlaneRow<LANES, R>::template load<POL_DEFAULT>(kept, make_rsrc(st, kExcessRange),
-                                                   in ? this->poff : kExcessDrop,
-                                                   lane_id() % LANES);
+                                                   in ? this->poff : kExcessDrop, this->ptail);
   }
 
   template <int JJ>
@@ -717,12 +717,12 @@ struct WinnerSearch {
   };
 
   static __device__ __forceinline__ void load(Row &r, const uint8_t *cost, const uint8_t *planes,
-                                              int coff, int poff, int Dp) {
+                                              int coff, int poff, int tail, int Dp) {
     bload_dwords<ND * CB, POL>(r.c, make_rsrc(cost, kExcessRange), coff);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(planes, kExcessRange);
 #pragma unroll
     for (int k = 0; k < NPL; k++)
-      PlaneRow<LANES, R>::template load<POL>(r.pl[k], rs, poff + k * Dp, lane_id() % LANES);
+      PlaneRow<LANES, R>::template load<POL>(r.pl[k], rs, poff + k * Dp, tail);
   }
 
   // Aggregates of one lane's cells, invalid and pad cells 0xFFFF.
@@ -798,6 +798,7 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner_kernel(PathJobs jobs
   const uint8_t *planes = V.planes + ((size_t)y * V.w + x0) * Dp * NPL;
   const int coff = inside ? (g * Dp + l * R) * CB : kExcessDrop;
   const int poff = inside ? g * NPL * Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
+  const int tail = PlaneRow<LANES, R>::tail(l);
   uint32_t kpk[NP];
 #pragma unroll
   for (int i = 0; i < NP; i++) {
@@ -807,14 +808,15 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner_kernel(PathJobs jobs
   uint8_t *row = cells[wv];
   const int own = lane * R * 2, line = g * LANES * R * 2;
   typename WS::Row cur;
-  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, Dp);
+  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, tail,
+           Dp);
   for (int i = 0; i < count; i += NL) {
     uint32_t S[NP];
     WS::sums(cur, beyond, paths, S);
     cost += NL * Dp * CB;
     planes += NL * Dp * NPL;
     const bool next = i + NL + g < count;
-    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, Dp);
+    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, tail, Dp);
 #pragma unroll
     for (int j = 0; j < NP; j += 2)
       *reinterpret_cast<uint2 *>(row + own + 4 * j) = make_uint2(S[j], S[j + 1]);
@@ -889,10 +891,12 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner32_kernel(PathJobs jo
   const uint8_t *planes = V.planes + ((size_t)y * V.w + x0) * Dp * 4;
   const int coff = inside ? (g * Dp + l * R) * 2 : kExcessDrop;
   const int poff = inside ? g * 4 * Dp + PlaneRow<LANES, R>::head(l) : kExcessDrop;
+  const int tail = PlaneRow<LANES, R>::tail(l);
   uint32_t *own = cells[wv] + lane * R;
   const uint32_t *line = cells[wv] + g * LANES * R;
   typename WS::Row cur;
-  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, Dp);
+  WS::load(cur, cost, planes, g < count ? coff : kExcessDrop, g < count ? poff : kExcessDrop, tail,
+           Dp);
   for (int i = 0; i < count; i += NL) {
     uint32_t S[R];  // invalid and pad cells: none
     uint32_t value = none;
@@ -909,7 +913,7 @@ __global__ __launch_bounds__(64 * kWinnerWaves) void winner32_kernel(PathJobs jo
     cost += NL * Dp * 2;
     planes += NL * Dp * 4;
     const bool next = i + NL + g < count;
-    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, Dp);
+    WS::load(cur, cost, planes, next ? coff : kExcessDrop, next ? poff : kExcessDrop, tail, Dp);
 #pragma unroll
     for (int j = 0; j < R; j += 4)
       *reinterpret_cast<uint4 *>(own + j) = make_uint4(S[j], S[j + 1], S[j + 2], S[j + 3]);
