@@ -792,14 +792,12 @@ void excess_codes(CostArgs &A) {
 }
 
 // Whether the band cost kernel (sgm_cost.h) takes the pair: a census-family
-// cost whose numerators stay below 2^31, a wave shape for the padded range, and
-// row segments of a wave within a 32-bit offset of each other.
-bool band_possible(const sgm_params *p, int w, int h) {
+// cost whose numerators stay below 2^31 and a wave shape for the padded range
+// (the row segments of a wave follow each other, so their offsets are small).
+bool band_possible(const sgm_params *p) {
   int lanes, R;
   const int Dp = padded_disparities(p->disparities);
-  if (p->cost > SGM_COST_CENSUS_GRADIENT || !excess_shape(Dp, lanes, R) ||
-      8 * (int64_t)std::max(w, h) * Dp >= (int64_t)1 << 30)
-    return false;
+  if (p->cost > SGM_COST_CENSUS_GRADIENT || !excess_shape(Dp, lanes, R)) return false;
   if (p->cost == SGM_COST_CENSUS) return true;
   const int64_t bits = p->window_w * p->window_h - 1;
   const int64_t cap = p->cost == SGM_COST_AD_CENSUS ? p->ad_truncation : p->gradient_truncation;
@@ -1063,11 +1061,13 @@ int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule, int
 // Whether the excess-plane kernels (sgm_excess.h) take the pair: excesses that
 // fit a byte (P2 <= 255), a wave shape for the padded range, and lines of a
 // wave whose rows lie within a 32-bit offset of each other.
-bool sgm::excess_possible(const sgm_params *p, int w, int h) {
+bool sgm::excess_possible(const sgm_params *p, int w) {
   int lanes, R;
   const int Dp = padded_disparities(p->disparities);
-  return effective_p2(p) <= 255 && excess_shape(Dp, lanes, R) &&
-         4 * (int64_t)std::max(w, h) * Dp * kMaxExcessDirs < (int64_t)1 << 30;
+  if (effective_p2(p) > 255 || !excess_shape(Dp, lanes, R)) return false;
+  // neighbouring lines start a row apart, two more round a corner of the image
+  const int64_t apart = lanes < 64 ? (int64_t)64 / lanes * w : 0;
+  return (apart + 1) * Dp * kMaxExcessDirs < (int64_t)kExcessRange;
 }
 
 // Whether a multi-direction schedule applies to the pair (budget aside).
@@ -1081,7 +1081,7 @@ bool sgm::schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, i
   if (!cost_volume || aggregate_bytes(p) != 2) return false;
   if (schedule == SGM_SWEEPS_PAIRED) return path_lanes(p) <= 8;
   return schedule == SGM_SWEEPS_PLANES && !ctx->keep_volumes && p->directions == kMaxExcessDirs &&
-         excess_possible(p, w, h) &&
+         excess_possible(p, w) &&
          (!cost_u8(p) || p->window_w * p->window_h - 1 + effective_p2(p) <= 255);
 }
 
@@ -1109,7 +1109,7 @@ int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h
   if (schedule == SGM_SWEEPS_PLANES)
     return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities),
                               plane_room(p, w, h, budget));
-  if (ctx->keep_volumes || !cost_volume || !excess_possible(p, w, h)) return 0;
+  if (ctx->keep_volumes || !cost_volume || !excess_possible(p, w)) return 0;
   if (schedule == SGM_SWEEPS_PAIRED) return p->directions == 4 ? 4 : 0;
   return aggregate_bytes(p) == 4 && ctx->sweeps != SGM_SWEEPS_SEQUENTIAL &&
                  (p->directions == 4 || 2 * effective_p2(p) <= 255)
@@ -2016,7 +2016,7 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
   const bool nt = (mode == 4 || mode == 1) && R <= 8 &&
                   (int64_t)nd * w * h * Dp * vol_bytes > (int64_t)768 << 20;
   if (nt) mode |= MODE_NT;
-  const bool band = !recompute && (B.nplanes || !fused) && band_possible(p, w, h);
+  const bool band = !recompute && (B.nplanes || !fused) && band_possible(p);
   if (!fused && !recompute && !band) {
     CostJobs cj;
     memset(&cj, 0, sizeof cj);

@@ -67,7 +67,7 @@ int64_t pair_bytes(const sgm_params *p, int w, int h);
 int64_t pair_bytes(const sgm_params *p, int w, int h, bool cost_volume);
 int64_t resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                            int schedule, bool fresh);
-bool excess_possible(const sgm_params *p, int w, int h);
+bool excess_possible(const sgm_params *p, int w);
 int excess_plane_count(const sgm_params *p, int64_t cells, int64_t room = INT64_MAX);
 int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                   bool cost_volume, int64_t budget);
@@ -129,7 +129,7 @@ int launch_path_pair(sgm_context *ctx, int R, int mode, int phase_b, const PathJ
                      const PathArgs &A, const PathJobs &jb, const PathArgs &B, int waves,
                      hipStream_t stream = nullptr);
 // census-family cost volumes (sgm_cost.h), on `stream` (the context's when null)
-bool band_possible(const sgm_params *p, int w, int h);
+bool band_possible(const sgm_params *p);
 int band_segment(const sgm_params *p, int64_t pixels);
 BandArgs band_args(const sgm_params *p, int njobs, bool excess);
 int launch_band(sgm_context *ctx, int Dp, const sgm_params *p, const PathJobs &jobs,
