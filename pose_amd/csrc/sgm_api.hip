@@ -1043,18 +1043,18 @@ struct PairBuffers {
 
 // Bytes that `budget` leaves for a resident pair's planes.
 static int64_t plane_room(const sgm_params *p, int w, int h, int64_t budget) {
-  const int64_t cells = 2 * (int64_t)w * h * padded_disparities(p->disparities);
-  return budget - (pair_bytes(p, w, h, true) - cells * aggregate_bytes(p));
+  return budget - (pair_bytes(p, w, h, true) - sweep_size(p, w, h).cells * aggregate_bytes(p));
 }
 
 // Device bytes a sweep schedule adds to pair_bytes(p, w, h, true): the second
 // partial aggregate volumes of paired sweeps, or the excess planes of both
 // matching directions (one byte per cell and plane) in place of the aggregates.
 int64_t sgm::schedule_bytes(const sgm_params *p, int w, int h, int schedule, int64_t budget) {
-  const int64_t cells = 2 * (int64_t)w * h * padded_disparities(p->disparities);
-  if (schedule == SGM_SWEEPS_PAIRED) return cells * aggregate_bytes(p);
+  const SweepSize size = sweep_size(p, w, h);
+  if (schedule == SGM_SWEEPS_PAIRED) return size.cells * aggregate_bytes(p);
   if (schedule == SGM_SWEEPS_PLANES)
-    return cells * (excess_plane_count(p, cells, plane_room(p, w, h, budget)) - aggregate_bytes(p));
+    return size.cells *
+           (excess_plane_count(p, size, plane_room(p, w, h, budget)) - aggregate_bytes(p));
   return 0;
 }
 
@@ -1085,17 +1085,46 @@ bool sgm::schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, i
          (!cost_u8(p) || p->window_w * p->window_h - 1 + effective_p2(p) <= 255);
 }
 
-// Planes per pixel of 8 paths over `cells` cells of all matching directions: one
-// per path, or one per pair of opposite paths (PairSweep, sgm_excess.h) where
-// their summed excesses fit a byte and the volumes are so far beyond the caches
-// that HBM traffic counts, or `room` bytes hold no more than the seven path-cost
-// planes that a budget may be sized for (640x480 D=64 in pairs 0.29 ms, with the
-// paired aggregates that would be next 0.73).
-int sgm::excess_plane_count(const sgm_params *p, int64_t cells, int64_t room) {
-  const bool far = cells * (1 + kMaxExcessDirs) > kPairBytes;
-  const bool tight = room >= cells * (kMaxExcessDirs - 1) && room < cells * kMaxExcessDirs;
+SweepSize sgm::sweep_size(const sgm_params *p, int w, int h) {
+  const int Dp = padded_disparities(p->disparities);
+  return {2 * (int64_t)w * h * Dp, std::max(w, h), std::min(w, h), Dp};
+}
+
+// Whether the steps of the longest lines set the time of the sweeps: images more than
+// twice as long as wide with fewer than `per_step` cells for each such step.
+static bool long_lines(const SweepSize &size, int64_t per_step) {
+  return size.longest > 2 * size.across && size.cells < per_step * size.longest;
+}
+
+// Planes per pixel of 8 paths: one per path, or one per pair of opposite paths
+// (PairSweep, sgm_excess.h) where their summed excesses fit a byte and
+//  - the volumes are so far beyond the caches that HBM traffic counts.  A pair sweep
+//    takes three steps in a row where a single sweep takes one, and the longer the
+//    more cells a lane holds, so not where long lines decide (Dp <= 512: above, the
+//    schedule that was is a chain of eight sweeps).  The line lies where both took the
+//    same: 4000x425 D=256 (218 thousand cells per step, line at 274) 4.5 ms in pairs,
+//    3.8 in single planes, 3000x566 (290) 3.6 and 3.8; D=64 (line at 106) 2500x680
+//    (87) 1.56 and 1.17; D=512 (line at 322) 8000x212 (217) 9.5 and 7.5, 4000x425
+//    (435) 6.9 and 7.6; or
+//  - `room` bytes hold no more than the seven path-cost planes that a budget may be
+//    sized for (640x480 D=64 in pairs 0.29 ms, with the paired aggregates that would
+//    be next 0.73).
+int sgm::excess_plane_count(const sgm_params *p, const SweepSize &size, int64_t room) {
+  int lanes = 64, R = 16;
+  excess_shape(size.Dp, lanes, R);
+  const int64_t per_step = 50000 + (lanes == 16 ? 14000 : 17000) * (int64_t)R;
+  const bool far = size.cells * (1 + kMaxExcessDirs) > kPairBytes &&
+                   !(size.Dp <= 512 && long_lines(size, per_step));
+  const bool tight = room >= size.cells * (kMaxExcessDirs - 1) && room < size.cells * kMaxExcessDirs;
   return 2 * effective_p2(p) <= 255 && (far || tight) ? kMaxExcessDirs / 2 : kMaxExcessDirs;
 }
+
+// Whether single planes of 16-bit sums are swept in narrow_shape.  16000x106 D=256 7.3
+// -> 4.3 ms a pair, 2500x680 4.0 -> 3.7, 8000x212 D=512 9.0 -> 7.5; with more cells per
+// step HBM decides and the wider waves' fewer instructions count (D=512: 435 thousand
+// 8.1 -> 7.6, 579 7.3 -> 8.0), and compact images have lines enough (250x187 D=192 116
+// -> 123 us).
+bool sgm::narrow_sweeps(const SweepSize &size) { return long_lines(size, 450000); }
 
 // Excess planes per pixel of a pair on the resident plan under `schedule` (0:
 // aggregate volumes).  With 4 paths the two partial aggregates of the paired
@@ -1106,15 +1135,21 @@ int sgm::excess_plane_count(const sgm_params *p, int64_t cells, int64_t room) {
 // cell replace 74 of eight sequential sweeps.
 int sgm::excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                        bool cost_volume, int64_t budget) {
+  const SweepSize size = sweep_size(p, w, h);
   if (schedule == SGM_SWEEPS_PLANES)
-    return excess_plane_count(p, 2 * (int64_t)w * h * padded_disparities(p->disparities),
-                              plane_room(p, w, h, budget));
+    return excess_plane_count(p, size, plane_room(p, w, h, budget));
   if (ctx->keep_volumes || !cost_volume || !excess_possible(p, w)) return 0;
   if (schedule == SGM_SWEEPS_PAIRED) return p->directions == 4 ? 4 : 0;
-  return aggregate_bytes(p) == 4 && ctx->sweeps != SGM_SWEEPS_SEQUENTIAL &&
-                 (p->directions == 4 || 2 * effective_p2(p) <= 255)
-             ? 4
-             : 0;
+  if (aggregate_bytes(p) != 4 || ctx->sweeps == SGM_SWEEPS_SEQUENTIAL) return 0;
+  if (p->directions == 4) return 4;
+  // long chains of the slowest steps (16 lanes of 12 cells and more, in pairs):
+  // 20000x15 D=256 21.8 ms against 15.3 of sequential sweeps, 1200x30 1.15 and 0.97,
+  // 16000x106 (54 thousand cells per step) 21.1 and 23.3; short ones are launches,
+  // 300x47 0.32 and 0.36
+  int lanes = 64, R = 16;
+  excess_shape(size.Dp, lanes, R);
+  const bool chain = lanes == 16 && R >= 12 && size.longest >= 512 && long_lines(size, 36000);
+  return 2 * effective_p2(p) <= 255 && !chain ? 4 : 0;
 }
 
 // Sweep schedule of a resident pair under `budget` (SGM_SWEEPS_SEQUENTIAL,
@@ -2108,6 +2143,8 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
     ExcessArgs E = excess_args(p, nd, B.nplanes);
     int lanes = 0, er = 0;
     excess_shape(Dp, lanes, er);
+    E.narrow = sb == 2 && !E.pairs && narrow_sweeps(sweep_size(p, w, h));
+    if (E.narrow) narrow_shape(Dp, lanes, er);
     const WaveLayout layout = wave_layout(E.ndirs, E.dx, E.dy, w, h, nd, 64 / lanes);
     memcpy(E.split, layout.split, sizeof E.split);
     memcpy(E.begin, layout.begin, sizeof E.begin);
@@ -2124,7 +2161,7 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
       return launch_winner32(ctx, Dp, stream, pj, WinnerArgs{p->directions, p->uniqueness}, w, h,
                              nd);
     return launch_winner(ctx, Dp, cost_bytes, B.nplanes, E.pairs ? 2 * E.p2 : E.p2, stream, pj,
-                         WinnerArgs{p->directions, p->uniqueness}, w, h, nd);
+                         WinnerArgs{p->directions, p->uniqueness}, w, h, nd, E.narrow);
   }
   // Paired sweeps: after the first direction, the middle directions run two
   // per launch, the first of each pair adding into the aggregate volume and

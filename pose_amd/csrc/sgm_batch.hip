@@ -85,11 +85,19 @@ static size_t group_table_bound(int count) {
 // in one device allocation.
 static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sgm_pair *pairs,
                         int count) {
-  // a group: one lane group R, under excess planes one wave shape of them
+  // a group: one lane group R, under excess planes one wave shape of them (and one
+  // of narrow sweeps)
+  auto lanes_of = [&](int Dp, int &R, bool narrow) {
+    int lanes = 0;
+    R = 0;
+    if (b->planes) excess_shape(Dp, lanes, R);
+    if (b->planes && narrow) narrow_shape(Dp, lanes, R);
+    return lanes;
+  };
   auto shape_of = [&](const PathJob &J) {
-    int lanes = 0, er = 0;
-    if (b->planes) excess_shape(J.Dp, lanes, er);
-    return std::make_pair(J.R, lanes * 64 + er);
+    int er, nr;
+    const int lanes = lanes_of(J.Dp, er, false), narrow = lanes_of(J.Dp, nr, b->narrow);
+    return std::make_pair(J.R, ((lanes * 64 + er) * 128 + narrow) * 64 + nr);
   };
   std::vector<std::pair<int, int>> rs;
   for (const PathJob &J : jobs)
@@ -110,7 +118,6 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     sgm_batch::Group g;
     g.R = R;
     g.sub = sub;
-    const int per = b->planes ? 64 / (key.second / 64) : 1;  // lines per wave
     std::vector<PathJob> gj;
     int64_t volume = 0, pixels = 0;
     bool aligned = true;
@@ -129,6 +136,10 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     }
     if (gj.empty()) continue;
     g.njobs = (int)gj.size();
+    // lines per wave of the sweeps, row segments per wave of the cost pass
+    int er;
+    const int per = b->planes ? 64 / lanes_of(g.Dp, er, b->narrow) : 1;
+    const int per_cost = b->planes ? 64 / lanes_of(g.Dp, er, false) : 1;
     sgm_params gp = b->params;
     gp.disparities = g.Dp;
     g.seg = band_segment(&gp, pixels);
@@ -146,7 +157,8 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
       for (size_t j = 0; j < gj.size(); j++) {
         const int n = cls == 3 ? gj[j].h * band_segments(gj[j].w, g.seg)
                                : lines_of(cls, gj[j].w, gj[j].h);
-        lb[j + 1] = lb[j] + (n + per - 1) / per;
+        const int k = cls == 3 ? per_cost : per;
+        lb[j + 1] = lb[j] + (n + k - 1) / k;
       }
       g.total_lines[cls] = lb.back();
       pd.lb_off[cls] = align_up(host.size(), 256);
@@ -289,6 +301,7 @@ static int phased_enqueue(sgm_batch *b) {
       A.stream = g.nt;
       if ((rc = launch_band(ctx, g.Dp, p, pj, A, st))) return rc;
       ExcessArgs E = excess_args(p, g.njobs, b->nplanes);
+      E.narrow = b->narrow;
       for (int k = 0; k < E.ndirs; k++) {
         E.begin[k] = E.total;
         E.total += g.total_lines[E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2];
@@ -297,7 +310,7 @@ static int phased_enqueue(sgm_batch *b) {
       E.order = g.order;
       if ((rc = launch_excess(ctx, g.Dp, 1, g.nt, pj, E, st))) return rc;
       if ((rc = launch_winner(ctx, g.Dp, 1, E.planes, E.pairs ? 2 * E.p2 : E.p2, g.nt, pj,
-                              WinnerArgs{p->directions, p->uniqueness}, g.w, g.h, g.njobs, st)))
+                              WinnerArgs{p->directions, p->uniqueness}, g.w, g.h, g.njobs, b->narrow, st)))
         return rc;
     }
     if ((rc = sync_streams(false))) return rc;
@@ -425,12 +438,26 @@ bool batch_planes_possible(const sgm_context *ctx, const sgm_params *params, con
   return true;
 }
 
+// All pairs of a batch as one: their cells, the longest line among them.
+static SweepSize batch_size(const sgm_params *params, const sgm_pair *pairs, int count) {
+  SweepSize all = {0, 0, 0, 64};
+  for (int i = 0; i < count; i++) {
+    sgm_params q = *params;
+    q.disparities = pairs[i].disparities;
+    const SweepSize s = sweep_size(&q, pairs[i].width, pairs[i].height);
+    all.cells += s.cells;
+    all.Dp = std::max(all.Dp, s.Dp);
+    if (s.longest > all.longest) {
+      all.longest = s.longest;
+      all.across = s.across;
+    }
+  }
+  return all;
+}
+
 // Excess planes per pixel of a batch.
 int batch_plane_count(const sgm_params *params, const sgm_pair *pairs, int count) {
-  int64_t cells = 0;
-  for (int i = 0; i < count; i++)
-    cells += 2 * (int64_t)pairs[i].width * pairs[i].height * padded_disparities(pairs[i].disparities);
-  return excess_plane_count(params, cells);
+  return excess_plane_count(params, batch_size(params, pairs, count));
 }
 
 // Scratch bytes of one pair under `nplanes` excess planes (carved as batch_create
@@ -550,6 +577,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
   b->pair_sub.assign(count, 0);
   if (planes != 0 && b->fused && batch_planes_possible(ctx, params, pairs, count, flags)) {
     b->nplanes = batch_plane_count(params, pairs, count);
+    b->narrow = b->nplanes == params->directions && narrow_sweeps(batch_size(params, pairs, count));
     size_t total = 0, largest = 0;
     for (int i = 0; i < count; i++) {
       total += batch_plane_bytes(pairs[i], b->nplanes);

@@ -91,6 +91,7 @@ struct sgm_batch {
   // plane blocks, each pair's sub-batch, and the sub-batch count
   bool planes = false;
   int nplanes = 0;  // excess planes per pixel
+  bool narrow = false;  // their sweeps in narrow_shape
   size_t scratch_bytes = 0;
   std::vector<int> pair_sub;
   int nsub = 1;

@@ -65,10 +65,23 @@ inline bool excess_shape(int Dp, int &lanes, int &R) {
   return true;
 }
 
+// The same with more lanes of fewer cells, for single planes of long images: a step of
+// a line is sooner done (0.18 against 0.28 us at 256 disparities), for more
+// instructions a cell.
+// false: none for these rows, lanes and R stay.
+inline bool narrow_shape(int Dp, int &lanes, int &R) {
+  const int u = Dp / 64;
+  if (u < 2 || u > 8) return false;
+  lanes = u == 2 ? 32 : 64;
+  R = u <= 4 ? 4 : 8;
+  return true;
+}
+
 struct ExcessArgs {
   int ndirs, total;      // directions (or pairs), wave slots over all of them
   int planes;            // plane rows per pixel
   int pairs;             // each entry sweeps a direction and its opposite
+  int narrow;            // narrow_shape
   int p1, p2, edge;
   int njobs;
   int dx[kMaxExcessDirs], dy[kMaxExcessDirs], begin[kMaxExcessDirs];

@@ -29,6 +29,14 @@ int launch_excess(sgm_context *ctx, int Dp, int cost_bytes, bool nt, const PathJ
   hipStream_t st = stream ? stream : ctx->stream;
   int lanes = 0, R = 0;
   if (excess_shape(Dp, lanes, R)) {
+    if (A.narrow && narrow_shape(Dp, lanes, R)) {
+#define CASE(L, RR)                                                          \
+  if (lanes == L && R == RR)                                                 \
+    return cost_bytes == 1 ? launch_excess_t<L, RR, 1, false>(st, nt, jobs, A) \
+                           : launch_excess_t<L, RR, 2, false>(st, nt, jobs, A);
+      CASE(32, 4) CASE(64, 4) CASE(64, 8)
+#undef CASE
+    }
     const bool pairs = A.pairs != 0;
 #define CASE(L, RR) \
   if (lanes == L && R == RR) return launch_excess_r<L, RR>(st, cost_bytes, pairs, nt, jobs, A);

@@ -68,7 +68,15 @@ int64_t pair_bytes(const sgm_params *p, int w, int h, bool cost_volume);
 int64_t resident_footprint(sgm_context *ctx, const sgm_params *p, int w, int h, bool cost_volume,
                            int schedule, bool fresh);
 bool excess_possible(const sgm_params *p, int w);
-int excess_plane_count(const sgm_params *p, int64_t cells, int64_t room = INT64_MAX);
+// What the choice of sweeps goes by: cells of all matching directions, the longest
+// line of an image and how many lie beside each other, padded disparities (the most)
+struct SweepSize {
+  int64_t cells;
+  int longest, across, Dp;
+};
+SweepSize sweep_size(const sgm_params *p, int w, int h);
+int excess_plane_count(const sgm_params *p, const SweepSize &size, int64_t room = INT64_MAX);
+bool narrow_sweeps(const SweepSize &size);
 int excess_planes(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
                   bool cost_volume, int64_t budget);
 bool schedule_applies(const sgm_context *ctx, const sgm_params *p, int w, int h, int schedule,
@@ -142,9 +150,9 @@ int launch_band16(hipStream_t st, int Dp, int words, bool diff, const PathJobs &
 int launch_excess(sgm_context *ctx, int Dp, int cost_bytes, bool nt, const PathJobs &jobs,
                   const ExcessArgs &A, hipStream_t stream = nullptr);
 // winner search over `planes` plane rows per pixel, each at most `largest`;
-// w, h: the largest image of the `njobs` jobs
+// w, h: the largest image of the `njobs` jobs; narrow: as the sweeps were
 int launch_winner(sgm_context *ctx, int Dp, int cost_bytes, int planes, int largest, bool nt,
-                  const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs,
+                  const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs, bool narrow,
                   hipStream_t stream = nullptr);
 // both for uint16 costs and four planes, in 32 bits
 int launch_excess32(sgm_context *ctx, int Dp, bool nt, const PathJobs &jobs, const ExcessArgs &A);

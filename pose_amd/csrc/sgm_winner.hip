@@ -28,7 +28,7 @@ static int launch_winner_r(hipStream_t st, int cost_bytes, int planes, int large
 }
 
 int launch_winner(sgm_context *ctx, int Dp, int cost_bytes, int planes, int largest, bool nt,
-                  const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs,
+                  const PathJobs &jobs, const WinnerArgs &A, int w, int h, int njobs, bool narrow,
                   hipStream_t stream) {
   ProfileScope ps(ctx, "path_winner");
   hipStream_t st = stream ? stream : ctx->stream;
@@ -36,6 +36,13 @@ int launch_winner(sgm_context *ctx, int Dp, int cost_bytes, int planes, int larg
   if ((planes != 4 && planes != 8) || !excess_shape(Dp, lanes, R))
     return fail(SGM_ERR_INVALID_ARGUMENT, "no winner search over %d planes of %d disparities",
                 planes, Dp);
+  // rows of 20 bytes a lane are split (PlaneRow) where the sweeps have that shape too;
+  // narrow sweeps leave 320 disparities in order
+  int narrow_lanes, narrow_R;
+  if (narrow && R == 20 && narrow_shape(Dp, narrow_lanes, narrow_R)) {
+    lanes = 32;
+    R = 16;
+  }
   constexpr int kMaxZ = 65535;  // grid z limit: jobs in slices
   for (int z0 = 0; z0 < njobs; z0 += kMaxZ) {
     const unsigned px = kWinnerPixels * kWinnerWaves;

@@ -1,5 +1,5 @@
-"""Excess-plane sweeps whose rows fill their padded length exactly, in every wave
-shape: the ranges whose rows leave lanes of a line idle (448, 576, 704, 832, 896 and
+"""Excess-plane sweeps whose rows fill their padded length exactly (and a few that do
+not), in every wave shape: the ranges whose rows leave lanes of a line idle (448, 576, 704, 832, 896 and
 960 disparities) have a real cell beside the idle lanes.  Single planes, pairs
 of opposite paths and 32-bit sums, in the caches and (volumes beyond 1 GiB) with
 the accesses that pass them; each equals the one-aggregate schedule bit for bit."""
@@ -15,14 +15,15 @@ SPARE = [448, 576, 704, 832, 896, 960]  # padded rows that leave lanes idle
 SHAPES = [64, 128, 192, 256, 320, 384, 512, 640, 768, 1024]  # one row per further shape
 
 
-def size_of(D, cells):
-    """A width past the range and the height that takes `cells` cells, both directions."""
-    w = max(D + 90, 700) | 1
-    return w, max(24, cells // (2 * w * D) + 1)
+def size_of(D, cells, wide):
+    """A width past the range and a height that takes `cells` cells, both directions;
+    up to 512 disparities at least half the width (longer images go by another rule)."""
+    w = (max(D + 90, 620) if cells else D + 60) | 1
+    return w, max(w // 2 + 1 if D <= 512 and not wide else 24, cells // (2 * w * D) + 1)
 
 
 # (name, D, cells of both directions, P2, bytes of a sum, planes, streamed)
-CASES = ([("pairs", D, GIB // 9, 120, 2, 4, False) for D in SPARE] +
+CASES = ([("pairs", D, GIB // 9, 120, 2, 4, False) for D in SPARE + [300, 350, 500]] +
          [("pairs streamed", D, GIB // 5, 120, 2, 4, True) for D in SPARE + SHAPES] +
          [("single", D, 0, 150, 2, 8, False) for D in SPARE] +
          [("single streamed", D, GIB // 9, 150, 2, 8, True) for D in SPARE + SHAPES] +
@@ -33,15 +34,16 @@ CASES = ([("pairs", D, GIB // 9, 120, 2, 4, False) for D in SPARE] +
 @pytest.mark.parametrize("case", CASES, ids=["%s-%d" % (c[0].replace(" ", "-"), c[1]) for c in CASES])
 def test_full_rows_equal_the_aggregate(case):
     name, D, cells, p2, sums, planes, streamed = case
-    w, h = size_of(D, cells)
+    w, h = size_of(D, cells, name.startswith("wide"))
     p = sgm.SgmParams(window_w=9, window_h=7, disparities=D, min_disparity=0, cost=0, p1=10, p2=p2,
                       edge_scale=32, directions=8, aggregate_bytes=sums, census_weight=500,
                       ad_truncation=30, gradient_truncation=60, reserved=0, uniqueness=0.03,
                       lr_threshold=1.0)
     cost = 1 if sums == 2 else 2
     # the rules on sizes that choose the planes and the cache policy
-    assert (2 * w * h * D * 9 > GIB and 2 * p2 <= 255) == (name.startswith("pairs")) or sums == 4
-    assert (2 * w * h * D * (cost + planes) > GIB) == streamed
+    padded = -(-D // 64) * 64
+    assert (2 * w * h * padded * 9 > GIB and 2 * p2 <= 255) == name.startswith("pairs") or sums == 4
+    assert (2 * w * h * padded * (cost + planes) > GIB) == streamed
     # most pixels near the top of the range, beside the idle lanes
     left, right, _ = synth.stereo_pair(w, h, D, 0, seed=D)
     shift = D - 2
