@@ -348,13 +348,14 @@ int sgm_set_cost_volume(sgm_context *ctx, int policy);
  *     direction.
  *   PLANES: a path cost is the cell's cost plus an excess of at most P2, so
  *     every direction, or pair of opposite directions (2 P2 <= 255, large
- *     pairs), stores its excesses as bytes into a plane of its own, all in one
+ *     pairs but long narrow ones), stores its excesses as bytes into a plane of its own, all in one
  *     launch (they only read the cost volume); the winner search adds the planes
  *     to the costs.  Needs P2 <= 255, for uint8 costs window bits - 1 + P2 <=
  *     255, 8 paths, at most 1024 padded disparities and no kept volumes; 8 or 4
  *     bytes per cell in place of the 2-byte aggregate, and 26 or 19 instead of
  *     36 bytes of HBM traffic per cell.  (4 paths under PAIRED: the room of the
- *     two partial aggregates holds one such plane per path.)
+ *     two partial aggregates holds one such plane per path; 32-bit sums: the room
+ *     of the int32 aggregate holds four, reported as SEQUENTIAL.)
  *   AUTO (default): PLANES where it applies and fits the budget, else PAIRED
  *     where that fits, else SEQUENTIAL.  A requested schedule that does not
  *     apply falls back the same way (PLANES -> PAIRED -> SEQUENTIAL). */
