@@ -817,6 +817,18 @@ int band_segment(const sgm_params *p, int64_t pixels) {
   return seg;
 }
 
+// Whether the band cost kernel pays for a call without planes: with few waves its row
+// segments, serial in their pixels, take longer than a thread per four cells.  Times of
+// both: AD-census 11x11, uint16, 100x40 D=320 41 and 13 us; level at about 20000 pixels
+// for D <= 320, 12000 for D=512, 8000 for D=1024, where the line lies or just below;
+// 226x141 0.86 (D=64) to 0.58 (D=1024) of it.  Kept volumes are for inspection and take
+// the kernel that larger images take; with planes the sweeps gained more than this.
+bool band_pays(const sgm_context *ctx, const sgm_params *p, int64_t pixels) {
+  int lanes = 64, R = 0;
+  excess_shape(padded_disparities(p->disparities), lanes, R);
+  return ctx->keep_volumes || pixels / 32 * lanes / 64 >= 192 + 5 * lanes;
+}
+
 // Arguments of the band cost kernel; the caller fills in the waves.  `excess`:
 // the volume codes of the excess-plane kernels.
 BandArgs band_args(const sgm_params *p, int njobs, bool excess) {
@@ -2051,7 +2063,8 @@ int run_directions(sgm_context *ctx, const sgm_params *p, int w, int h, PairBuff
   const bool nt = (mode == 4 || mode == 1) && R <= 8 &&
                   (int64_t)nd * w * h * Dp * vol_bytes > (int64_t)768 << 20;
   if (nt) mode |= MODE_NT;
-  const bool band = !recompute && (B.nplanes || !fused) && band_possible(p);
+  const bool band = !recompute && band_possible(p) &&
+                    (B.nplanes || (!fused && band_pays(ctx, p, (int64_t)nd * w * h)));
   if (!fused && !recompute && !band) {
     CostJobs cj;
     memset(&cj, 0, sizeof cj);
