@@ -781,14 +781,13 @@ CostArgs cost_args(const sgm_params *p) {
   A.gradcap = p->gradient_truncation;
   A.inv_code = invalid_code(p);
   A.u8 = cost_u8(p) ? 1 : 0;
-  A.inv_store = A.pad_store = A.u8 ? 255 : A.inv_code;
   return A;
 }
 
-// Volume codes of the excess-plane kernels (sgm_excess.h).
-void excess_codes(CostArgs &A) {
-  A.inv_store = A.u8 ? 254 : 0x8000 | A.inv_code;
-  A.pad_store = A.u8 ? 255 : 0x8FFF;
+// Volume codes; `excess`: those of the excess-plane kernels (sgm_excess.h).
+CostCodes cost_codes(const CostArgs &A, bool excess) {
+  if (!excess) return A.u8 ? CostCodes{255, 255} : CostCodes{A.inv_code, A.inv_code};
+  return A.u8 ? CostCodes{254, 255} : CostCodes{0x8000 | A.inv_code, 0x8FFF};
 }
 
 // Whether the band cost kernel (sgm_cost.h) takes the pair: a census-family
@@ -845,11 +844,11 @@ BandArgs band_args(const sgm_params *p, int njobs, bool excess) {
     A.half = 1000 * A.cap / 2;
     band_division(1000 * A.cap, A.magic, A.shift);
   }
-  CostArgs C = cost_args(p);
-  if (excess) excess_codes(C);
+  const CostArgs C = cost_args(p);
+  const CostCodes S = cost_codes(C, excess);
   const uint32_t rep = C.u8 ? 0x01010101u : 0x00010001u;
-  A.inv = (uint32_t)C.inv_store * rep;
-  A.pad = (uint32_t)C.pad_store * rep;
+  A.inv = (uint32_t)S.inv * rep;
+  A.pad = (uint32_t)S.pad * rep;
   return A;
 }
 
@@ -868,11 +867,8 @@ int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h,
                 const sgm_params *p, int rows, bool force_u16, bool excess) {
   ProfileScope ps(ctx, "cost");
   CostArgs A = cost_args(p);
-  if (force_u16) {
-    A.u8 = 0;
-    A.inv_store = A.pad_store = A.inv_code;
-  }
-  if (excess) excess_codes(A);
+  if (force_u16) A.u8 = 0;
+  const CostCodes S = cost_codes(A, excess);
   const int gy = rows < 0 ? h : rows;
   if (p->cost == SGM_COST_ZNCC || p->cost == SGM_COST_ZNCC_FP32) {
     const int ntx = (w + kZnccTX - 1) / kZnccTX, ntd = (Dp + 63) / 64;
@@ -881,11 +877,11 @@ int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h,
 #define ZNCC_LAUNCH(RR)                                                                   \
   case RR:                                                                                \
     if (p->cost == SGM_COST_ZNCC_FP32)                                                    \
-      zncc_band_kernel<RR, 4, false><<<grid, 64, 0, ctx->stream>>>(jobs, A, gy);          \
+      zncc_band_kernel<RR, 4, false><<<grid, 64, 0, ctx->stream>>>(jobs, A, S, gy);          \
     else if (out8)                                                                        \
-      zncc_band_kernel<RR, 3, true><<<grid, 64, 0, ctx->stream>>>(jobs, A, gy);           \
+      zncc_band_kernel<RR, 3, true><<<grid, 64, 0, ctx->stream>>>(jobs, A, S, gy);           \
     else                                                                                  \
-      zncc_band_kernel<RR, 3, false><<<grid, 64, 0, ctx->stream>>>(jobs, A, gy);          \
+      zncc_band_kernel<RR, 3, false><<<grid, 64, 0, ctx->stream>>>(jobs, A, S, gy);          \
     break;
     switch (p->window_w / 2) {
       ZNCC_LAUNCH(1) ZNCC_LAUNCH(2) ZNCC_LAUNCH(3) ZNCC_LAUNCH(4) ZNCC_LAUNCH(5)
@@ -897,7 +893,7 @@ int launch_cost(sgm_context *ctx, const CostJobs &jobs, int njobs, int w, int h,
   }
   const int quads = w * (Dp / 4);
   dim3 grid((quads + 255) / 256, gy, njobs);
-  cost_kernel<<<grid, 256, 0, ctx->stream>>>(jobs, A);
+  cost_kernel<<<grid, 256, 0, ctx->stream>>>(jobs, A, S);
   return launch_check("cost kernel");
 }
 

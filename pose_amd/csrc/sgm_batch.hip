@@ -211,22 +211,6 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
   return SGM_OK;
 }
 
-// One launch of the work-queue kernel over items [lo, hi) with its own head.
-static int queue_launch(sgm_batch *b, int lo, int hi, unsigned *head, const char *what) {
-  if (hi <= lo) return SGM_OK;
-  BatchArgs A = b->args;
-  A.item_lo = lo;
-  A.item_hi = hi;
-  A.head = head;
-  A.phased = 1;
-  ProfileScope ps(b->ctx, what);
-  void *kargs[] = {(void *)&A};
-  hipError_t e = hipLaunchKernel(batch_kernel_of(b), dim3((unsigned)b->blocks),
-                                 dim3(b->waves_per_block * 64), kargs, 0, b->stream);
-  if (e == hipSuccess) e = hipGetLastError();
-  return e == hipSuccess ? SGM_OK : hip_fail(e, "batch kernel launch");
-}
-
 // Census (lr = false) or L-R (lr = true) phase of a phase-major run as one
 // regular grid over every image or pair: 64-column tiles of row bands, four
 // per block (a queue item is a whole row band, too few waves for a few pairs).
@@ -252,7 +236,25 @@ static int grid_launch(sgm_batch *b, bool lr) {
   return SGM_OK;
 }
 
-// Phase-major run: the census grid (and the cost items), the sweeps direction
+// The cost phase (non-fused costs) of a phase-major run.
+static int cost_launch(sgm_batch *b) {
+  int h = 1;
+  for (const sgm_pair &pr : b->pairs) h = std::max(h, pr.height);
+  const int n = (int)b->pairs.size() * 2;
+  constexpr int kMaxZ = 65535;  // grid z limit: jobs in slices
+  ProfileScope ps(b->ctx, "batch cost");
+  for (int z0 = 0; z0 < n; z0 += kMaxZ) {
+    const dim3 grid((unsigned)h, 1, (unsigned)std::min(kMaxZ, n - z0));
+    // ZNCC costs only use uint16 volumes, as in batch_kernel
+    if (b->cost8) batch_cost_grid<false><<<grid, 64 * kGridWaves, 0, b->stream>>>(b->args, z0);
+    else batch_cost_grid<true><<<grid, 64 * kGridWaves, 0, b->stream>>>(b->args, z0);
+    int rc = launch_check("batch cost grid");
+    if (rc) return rc;
+  }
+  return SGM_OK;
+}
+
+// Phase-major run: the census grid (and the cost grid), the sweeps direction
 // by direction and lane group by lane group with the specialised sweep kernel,
 // the L-R grid.
 static int phased_enqueue(sgm_batch *b) {
@@ -261,9 +263,7 @@ static int phased_enqueue(sgm_batch *b) {
   const std::vector<int> &pb = b->phase_begin;
   int rc;
   if ((rc = grid_launch(b, false))) return rc;
-  // cost items (non-fused costs) after the census grid: their waits on the
-  // census phase pass at once, an earlier launch having run it
-  if ((rc = queue_launch(b, pb[BPH_COST], pb[BPH_PATH0], b->args.head, "batch cost"))) return rc;
+  if (pb[BPH_PATH0] > pb[BPH_COST] && (rc = cost_launch(b))) return rc;
   const int sb = b->sum_bytes;
   if (b->planes) {
     // excess planes, sub-batch after sub-batch (one scratch region): per group
@@ -716,7 +716,14 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
   std::vector<CostJob> cjobs(2 * count);
   std::vector<BatchPairDev> pdev(count);
   b->slots.resize(count);
-  const int census_rows = kBatchCensusRows, cost_rows = 4, lr_rows = 16;
+  // rows of a cost item: four (64 pairs of 320x240 D=64 with AD-census costs 31.9 ms, one
+  // by one 32.3) where every wave gets several of them, else one (three gradient pairs up
+  // to 700x500, D up to 400, 8 paths: 4.7 ms -> 3.6, larger ones and 4 paths 11.7 -> 5.9;
+  // seven ZNCC pairs 72 -> 25)
+  int64_t cost_lines = 0;
+  for (int i = 0; i < count; i++) cost_lines += 2 * (int64_t)pairs[i].height;
+  const int64_t waves = (int64_t)b->blocks * b->waves_per_block;
+  const int census_rows = kBatchCensusRows, cost_rows = cost_lines >= 4 * waves ? 4 : 1, lr_rows = 16;
   std::vector<int> job_begin((size_t)nph * stride, 0), phase_begin(nph + 1, 0);
   auto P8 = [&](size_t o) { return base + o; };
   for (int i = 0; i < count; i++) {
@@ -891,9 +898,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
   A.ww = params->window_w;
   A.wh = params->window_h;
   A.lr_threshold = params->lr_threshold;
-  A.item_lo = 0;
-  A.item_hi = total;
-  A.phased = 0;
+  A.items = total;
   if (flags & SGM_BATCH_PHASED) {
     if ((rc = build_groups(b, jobs, pairs, count))) {
       sgm_batch_destroy(b);

@@ -57,11 +57,7 @@ struct BatchArgs {
   int ww, wh;
   double lr_threshold;
   long long spin_limit;    // wall-clock ticks a dependency wait may take before the error flag
-  // the queue range of this launch; a phase-major run launches the census /
-  // cost phases and the L-R phase separately (the sweeps run between them),
-  // and phases that end before item_lo were completed by earlier launches
-  int item_lo, item_hi;
-  int phased;
+  int items;               // queue items of all phases
 };
 
 __device__ __forceinline__ int batch_phase_of(const BatchArgs &B, int item) {
@@ -95,7 +91,6 @@ __device__ __forceinline__ int batch_njobs(const BatchArgs &B, int ph) {
 // invalidation per iteration); the caller issues one acquire fence after the
 // wait succeeds.
 __device__ __forceinline__ bool batch_wait(const BatchArgs &B, int ph, int job) {
-  if (B.phased && B.phase_begin[ph] < B.item_lo) return true;  // an earlier launch ran it
   const unsigned need = (unsigned)batch_items(B, ph, job);
   unsigned *ctr = B.done + (size_t)ph * B.stride + job;
   if (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= need) return true;
@@ -178,15 +173,16 @@ __device__ __forceinline__ void batch_census(const BatchArgs &B, const BatchImag
   for (int x0 = 0; x0 < I.w; x0 += 64) batch_census_chunk<WORDS>(B, I, x0, r0, r1, tile);
 }
 
-// Cost volume rows [r0, r1) of one matching direction (non-fused costs).
+// Cost volume rows [r0, r1) of one matching direction (non-fused costs), `step`
+// threads to a row of which this is number `first`.
 template <bool ZNCC>
-__device__ __forceinline__ void batch_cost(const BatchArgs &B, const CostJob &J, int r0, int r1) {
-  const int lane = lane_id();
+__device__ __forceinline__ void batch_cost(const BatchArgs &B, const CostJob &J, int r0, int r1,
+                                           int first, int step) {
   const int rx = B.ww >> 1, ry = B.wh >> 1;
   const size_t n = (size_t)J.w * J.h;
   const int quads = J.Dp >> 2;
   for (int y = r0; y < r1; y++) {
-    for (int qi = lane; qi < J.w * quads; qi += 64) {
+    for (int qi = first; qi < J.w * quads; qi += step) {
       const int x = qi / quads, k0 = (qi - x * quads) * 4;
       const size_t p = (size_t)y * J.w + x;
       const bool pix_ok = x >= rx && x < J.w - rx && y >= ry && y < J.h - ry && J.mask_a[p];
@@ -344,7 +340,7 @@ void batch_kernel(BatchArgs B) {
   __syncthreads();
   const int lane = lane_id(), wave = threadIdx.x >> 6;
   uint8_t *tile = tiles[wave];
-  const int total = B.item_hi;
+  const int total = B.items;
   static const int dirs[8][2] = {{1, 0}, {-1, 0}, {0, 1}, {0, -1}, {1, 1}, {-1, 1}, {1, -1}, {-1, -1}};
   // Completions of the current (phase, job) run are published together, before
   // the wave waits on anything else, so no wave waits while holding them.
@@ -354,7 +350,7 @@ void batch_kernel(BatchArgs B) {
   for (;;) {
     int got = 0;
     if (lane == 0) got = (int)atomicAdd(B.head, 1u);
-    const int item = B.item_lo + __builtin_amdgcn_readlane(got, 0);
+    const int item = __builtin_amdgcn_readlane(got, 0);
     if (item >= total) break;
     const int ph = batch_phase_of(B, item);
     const int nj = batch_njobs(B, ph);
@@ -395,7 +391,7 @@ void batch_kernel(BatchArgs B) {
     } else if (ph == BPH_COST) {
       const CostJob J = B.cost_jobs[job];
       const int r0 = tile_idx * B.cost_rows, r1 = min(J.h, r0 + B.cost_rows);
-      batch_cost<VOL == VOL_U16>(B, J, r0, r1);  // ZNCC costs only use uint16 volumes
+      batch_cost<VOL == VOL_U16>(B, J, r0, r1, lane, 64);  // ZNCC costs only use uint16 volumes
     } else if (ph <= last_path) {
       const PathJob J = B.jobs[job];
       const int dir = ph - BPH_PATH0;
@@ -436,6 +432,18 @@ static __global__ __launch_bounds__(256) void batch_census_grid(BatchArgs B, int
   const int x0 = (blockIdx.x * kGridWaves + wave) * 64, r0 = blockIdx.y * kBatchCensusRows;
   if (x0 >= I.w || r0 >= I.h) return;  // wave-uniform: the tile lies outside this image
   batch_census_chunk<WORDS>(B, I, x0, r0, min(I.h, r0 + kBatchCensusRows), tiles[wave]);
+}
+
+// The cost phase (non-fused costs) of phase-major runs: a block per row of a job, so
+// that a few pairs fill the chip.  Bound by the cells' arithmetic (a division each,
+// or the window of a ZNCC cost).  As items of batch_kernel, four rows to a wave and
+// among that kernel's spilled scalars, the AD-census costs of 321x152 D=493, 47x1055
+// D=448, 324x121 D=256 and 236x236 D=320 took 4.0 to 4.4 ms, so 0.40.
+template <bool ZNCC>
+static __global__ __launch_bounds__(256) void batch_cost_grid(BatchArgs B, int z0) {
+  const CostJob J = B.cost_jobs[z0 + (int)blockIdx.z];
+  const int y = blockIdx.x;
+  if (y < J.h) batch_cost<ZNCC>(B, J, y, y + 1, threadIdx.x, 64 * kGridWaves);
 }
 
 static __global__ __launch_bounds__(256) void batch_lr_grid(BatchArgs B, int z0) {

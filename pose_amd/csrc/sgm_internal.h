@@ -121,7 +121,7 @@ int64_t esgm_pair_bytes(const sgm_params *p, int w, int h, int rows, int pool);
 const char *esgm_unsupported(const sgm_params *p, int w, int h);
 int esgm_plan(sgm_context *ctx, const sgm_params *p, int w, int h, int *rows, int *pool);
 CostArgs cost_args(const sgm_params *p);
-void excess_codes(CostArgs &A);
+CostCodes cost_codes(const CostArgs &A, bool excess);
 ExcessArgs excess_args(const sgm_params *p, int njobs, int planes);
 // volumes beyond this stream past the caches (far more than the 256 MB MALL)
 constexpr int64_t kStreamBytes = (int64_t)1 << 30;

@@ -233,8 +233,12 @@ struct CostJob {
 struct CostArgs {
   int mode, ww, wh, words, weight, adcap, gradcap, inv_code;
   int u8;  // uint8 cost volume (census-family costs <= 120, 255 = invalid 512)
-  // codes of an invalid cell and of a pad cell (k >= D) as stored in the volume
-  int inv_store, pad_store;
+};
+// Codes of an invalid cell and of a pad cell (k >= D) as stored in the volume (apart
+// from CostArgs: the batch kernel carries those, and two more words there cost it 300
+// spilled SGPRs and 9% of its cost phase).
+struct CostCodes {
+  int inv, pad;
 };
 
 // Stores the costs of disparities k0 .. k0+3 of pixel p.
@@ -387,7 +391,8 @@ __device__ __forceinline__ int zncc_px(const uint8_t *img, int w, int row, int x
 }
 
 template <int RX, int MODE, bool REV, bool OUT8>
-__device__ __forceinline__ void zncc_band(const CostJob &J, const CostArgs &A, int rows) {
+__device__ __forceinline__ void zncc_band(const CostJob &J, const CostArgs &A, const CostCodes &S,
+                                          int rows) {
   constexpr int XW = kZnccTX + 2 * RX;  // window columns of one tile
   const int ntx = (J.w + kZnccTX - 1) / kZnccTX;
   const int x0 = (int)(blockIdx.x % ntx) * kZnccTX;
@@ -510,8 +515,8 @@ __device__ __forceinline__ void zncc_band(const CostJob &J, const CostArgs &A, i
         c = c > -1.0 ? c : -1.0;
         value = ok ? (int)round_half_up_d((1.0 - c) * .5 * bits) : 512;
       }
-      if (MODE != 4) value = value == 512 ? A.inv_store : value;
-      value = kin ? value : A.pad_store;
+      if (MODE != 4) value = value == 512 ? S.inv : value;
+      value = kin ? value : S.pad;
       if (kst) {
         if (OUT8) out[(size_t)xo * ostep] = (uint8_t)value;
         else *(uint16_t *)(out + (size_t)xo * ostep) = (uint16_t)value;
@@ -530,13 +535,14 @@ __device__ __forceinline__ void zncc_band(const CostJob &J, const CostArgs &A, i
 // direction of the target side is fixed per job, so each block takes one
 // branch at entry and the cell loop stays branch-free.
 template <int RX, int MODE, bool OUT8>
-static __global__ __launch_bounds__(64) void zncc_band_kernel(CostJobs jobs, CostArgs A, int rows) {
+static __global__ __launch_bounds__(64) void zncc_band_kernel(CostJobs jobs, CostArgs A, CostCodes S,
+                                                              int rows) {
   const CostJob &J = jobs.job[blockIdx.z];
-  if (J.reverse) zncc_band<RX, MODE, true, OUT8>(J, A, rows);
-  else zncc_band<RX, MODE, false, OUT8>(J, A, rows);
+  if (J.reverse) zncc_band<RX, MODE, true, OUT8>(J, A, S, rows);
+  else zncc_band<RX, MODE, false, OUT8>(J, A, S, rows);
 }
 
-static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArgs A) {
+static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArgs A, CostCodes S) {
   const CostJob J = jobs.job[blockIdx.z];
   const int y = blockIdx.y + J.y0;
   if (y >= J.h) return;
@@ -551,7 +557,7 @@ static __global__ __launch_bounds__(256) void cost_kernel(CostJobs jobs, CostArg
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int k = k0 + j;
-    int value = k < J.D ? A.inv_store : A.pad_store;
+    int value = k < J.D ? S.inv : S.pad;
     if (pix_ok && k < J.D) {
       const int disp = J.minD + k;
       const long long t = (long long)x + (J.reverse ? (long long)disp : -(long long)disp);
