@@ -85,8 +85,11 @@ static size_t group_table_bound(int count) {
 // in one device allocation.
 static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sgm_pair *pairs,
                         int count) {
-  // a group: one lane group R, under excess planes one wave shape of them (and one
-  // of narrow sweeps)
+  // a group: one lane group R, under excess planes one wave shape
+  auto narrow_of = [&](const PathJob &J) {
+    return b->planes && b->nplanes == b->params.directions &&
+           narrow_sweeps(SweepSize{b->cells, std::max(J.w, J.h), std::min(J.w, J.h), J.Dp});
+  };
   auto lanes_of = [&](int Dp, int &R, bool narrow) {
     int lanes = 0;
     R = 0;
@@ -94,10 +97,11 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     if (b->planes && narrow) narrow_shape(Dp, lanes, R);
     return lanes;
   };
+  // (the cost pass and the winner take the ordinary shape, the sweeps their own)
   auto shape_of = [&](const PathJob &J) {
     int er, nr;
-    const int lanes = lanes_of(J.Dp, er, false), narrow = lanes_of(J.Dp, nr, b->narrow);
-    return std::make_pair(J.R, ((lanes * 64 + er) * 128 + narrow) * 64 + nr);
+    const int lanes = lanes_of(J.Dp, er, false), own = lanes_of(J.Dp, nr, narrow_of(J));
+    return std::make_pair(J.R, ((lanes * 64 + er) * 128 + own) * 64 + nr);
   };
   std::vector<std::pair<int, int>> rs;
   for (const PathJob &J : jobs)
@@ -130,6 +134,7 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
         aligned &= J.Dp % 64 == 0;
         pixels += (int64_t)J.w * J.h;
         g.Dp = J.Dp;
+        g.narrow = narrow_of(J);
         g.w = std::max(g.w, J.w);
         g.h = std::max(g.h, J.h);
       }
@@ -138,7 +143,7 @@ static int build_groups(sgm_batch *b, const std::vector<PathJob> &jobs, const sg
     g.njobs = (int)gj.size();
     // lines per wave of the sweeps, row segments per wave of the cost pass
     int er;
-    const int per = b->planes ? 64 / lanes_of(g.Dp, er, b->narrow) : 1;
+    const int per = b->planes ? 64 / lanes_of(g.Dp, er, g.narrow) : 1;
     const int per_cost = b->planes ? 64 / lanes_of(g.Dp, er, false) : 1;
     sgm_params gp = b->params;
     gp.disparities = g.Dp;
@@ -301,7 +306,7 @@ static int phased_enqueue(sgm_batch *b) {
       A.stream = g.nt;
       if ((rc = launch_band(ctx, g.Dp, p, pj, A, st))) return rc;
       ExcessArgs E = excess_args(p, g.njobs, b->nplanes);
-      E.narrow = b->narrow;
+      E.narrow = g.narrow;
       for (int k = 0; k < E.ndirs; k++) {
         E.begin[k] = E.total;
         E.total += g.total_lines[E.dy[k] == 0 ? 0 : E.dx[k] == 0 ? 1 : 2];
@@ -310,7 +315,7 @@ static int phased_enqueue(sgm_batch *b) {
       E.order = g.order;
       if ((rc = launch_excess(ctx, g.Dp, 1, g.nt, pj, E, st))) return rc;
       if ((rc = launch_winner(ctx, g.Dp, 1, E.planes, E.pairs ? 2 * E.p2 : E.p2, g.nt, pj,
-                              WinnerArgs{p->directions, p->uniqueness}, g.w, g.h, g.njobs, b->narrow, st)))
+                              WinnerArgs{p->directions, p->uniqueness}, g.w, g.h, g.njobs, g.narrow, st)))
         return rc;
     }
     if ((rc = sync_streams(false))) return rc;
@@ -577,7 +582,7 @@ int batch_create(sgm_context *ctx, const sgm_params *params, const sgm_pair *pai
   b->pair_sub.assign(count, 0);
   if (planes != 0 && b->fused && batch_planes_possible(ctx, params, pairs, count, flags)) {
     b->nplanes = batch_plane_count(params, pairs, count);
-    b->narrow = b->nplanes == params->directions && narrow_sweeps(batch_size(params, pairs, count));
+    b->cells = batch_size(params, pairs, count).cells;
     size_t total = 0, largest = 0;
     for (int i = 0; i < count; i++) {
       total += batch_plane_bytes(pairs[i], b->nplanes);

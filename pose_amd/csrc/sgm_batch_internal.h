@@ -76,6 +76,7 @@ struct sgm_batch {
   struct Group {
     int R = 0, njobs = 0, sub = 0;
     bool nt = false;
+    bool narrow = false;  // excess sweeps in narrow_shape
     const sgm::PathJob *jobs = nullptr;
     int Dp = 0, w = 0, h = 0;  // padded disparities of a job, largest sizes
     int seg = 128;             // pixels per row segment of the cost pass
@@ -91,7 +92,7 @@ struct sgm_batch {
   // plane blocks, each pair's sub-batch, and the sub-batch count
   bool planes = false;
   int nplanes = 0;  // excess planes per pixel
-  bool narrow = false;  // their sweeps in narrow_shape
+  int64_t cells = 0;  // cells of every pair, both matching directions
   size_t scratch_bytes = 0;
   std::vector<int> pair_sub;
   int nsub = 1;

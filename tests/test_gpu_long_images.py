@@ -3,6 +3,8 @@ in the narrow wave shapes, not planes of pairs; sequential 32-bit sweeps where t
 pairs' chain would be longer; widths past 65535.  Results equal the one-aggregate
 schedule bit for bit, alone and in phase-major batches, and the choice is no slower
 than that schedule."""
+import time
+
 import numpy as np
 import pytest
 
@@ -123,3 +125,36 @@ def test_long_images_in_a_batch(graph):
                 x.free()
     finally:
         ctx.close()
+
+
+def test_ordinary_pairs_beside_a_long_one_keep_their_shape():
+    # the narrow waves of one long image are not taken to the others, which take
+    # no longer with it beside them than both by themselves
+    sizes = [(4000, 60, 128), (640, 480, 128), (640, 480, 128)]
+
+    def run(sizes):
+        ctx = sgm.Context(0)
+        try:
+            records = []
+            for i, (w, h, D) in enumerate(sizes):
+                left, right, _ = synth.stereo_pair(w, h, D, 0, seed=80 + i)
+                n = w * h
+                b = [ctx.alloc(n).upload(left), ctx.alloc(n).upload(right), ctx.alloc(4 * n)]
+                records.append(sgm.SgmPair(width=w, height=h, disparities=D, min_disparity=0,
+                                           left=b[0].ptr, right=b[1].ptr, checked=b[2].ptr))
+            batch = sgm.DeviceBatch(ctx, params(64), records, phased=True)
+            least = 1e9
+            for _ in range(8):
+                ctx.synchronize()
+                start = time.perf_counter()
+                batch.run()
+                ctx.synchronize()
+                least = min(least, time.perf_counter() - start)
+            batch.close()
+            return 1e3 * least
+        finally:
+            ctx.close()
+
+    together, long, others = run(sizes), run(sizes[:1]), run(sizes[1:])
+    print("long batch ms", together, "long", long, "others", others, flush=True)
+    assert together <= 1.05 * (long + others)
