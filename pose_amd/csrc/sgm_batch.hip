@@ -249,7 +249,8 @@ static int cost_launch(sgm_batch *b) {
   constexpr int kMaxZ = 65535;  // grid z limit: jobs in slices
   ProfileScope ps(b->ctx, "batch cost");
   for (int z0 = 0; z0 < n; z0 += kMaxZ) {
-    const dim3 grid((unsigned)h, 1, (unsigned)std::min(kMaxZ, n - z0));
+    // (a launch holds fewer than 2^32 threads along x: taller images take turns)
+    const dim3 grid((unsigned)std::min(h, 1 << 20), 1, (unsigned)std::min(kMaxZ, n - z0));
     // ZNCC costs only use uint16 volumes, as in batch_kernel
     if (b->cost8) batch_cost_grid<false><<<grid, 64 * kGridWaves, 0, b->stream>>>(b->args, z0);
     else batch_cost_grid<true><<<grid, 64 * kGridWaves, 0, b->stream>>>(b->args, z0);

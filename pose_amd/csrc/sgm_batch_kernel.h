@@ -442,8 +442,8 @@ static __global__ __launch_bounds__(256) void batch_census_grid(BatchArgs B, int
 template <bool ZNCC>
 static __global__ __launch_bounds__(256) void batch_cost_grid(BatchArgs B, int z0) {
   const CostJob J = B.cost_jobs[z0 + (int)blockIdx.z];
-  const int y = blockIdx.x;
-  if (y < J.h) batch_cost<ZNCC>(B, J, y, y + 1, threadIdx.x, 64 * kGridWaves);
+  for (int y = blockIdx.x; y < J.h; y += (int)gridDim.x)
+    batch_cost<ZNCC>(B, J, y, y + 1, threadIdx.x, 64 * kGridWaves);
 }
 
 static __global__ __launch_bounds__(256) void batch_lr_grid(BatchArgs B, int z0) {
